@@ -25,6 +25,12 @@
  *                   over the first power-of-two count of groups that covers
  *                   every group with a lane still running (one graph per
  *                   count), so finished groups cost nothing.
+ *                   Once a handle's cycles pay for the planning (about one
+ *                   cycle per 512 gates), netlists whose live planes fit a
+ *                   workgroup's LDS at 8, 16 or 32 stimuli per workgroup run
+ *                   there instead: whole runs in one kernel, live gates only,
+ *                   each workgroup to its own longest budget. The hashes are
+ *                   the same.
  *
  * No counterpart in the reference, which compiles every design through its
  * emitter (src/V3EmitC.cpp); the protocol and hash are the benchmark's.
@@ -53,7 +59,8 @@ int rf_gn_create(const uint32_t* program, size_t words, uint32_t n_lanes, rf_gat
 int rf_gn_run(rf_gatenet* g, uint32_t mode, uint64_t seed, const uint32_t* budgets,
               uint64_t* out_hashes, float* ms);
 
-/* Mtasks of the loaded partition, graph nodes per clock cycle of a mode. */
+/* Mtasks of the loaded partition, graph nodes per clock cycle of a mode (0
+ * before its first run, and for RF_GN_BITPLANE once it runs in LDS). */
 uint32_t rf_gn_mtasks(const rf_gatenet* g);
 uint32_t rf_gn_nodes_per_cycle(const rf_gatenet* g, uint32_t mode);
 

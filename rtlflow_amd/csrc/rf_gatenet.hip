@@ -23,6 +23,8 @@
 #include <vector>
 
 #include "rf_gatenet.h"
+#include "rf_gnlds.h"
+#include "rf_gnplan.h"
 #include "rf_stim.h"
 #include "rf_transpose.h"
 #include "rf_verilated.h"
@@ -31,15 +33,10 @@ int rf_set_error(int code, const char* fmt, ...);
 
 namespace {
 
-enum {
-    H_MAGIC, H_VERSION, H_NODES, H_PI, H_FF, H_RAMBITS, H_PO, H_RAMS, H_DEPTH, H_WIDTH, H_ABITS,
-    H_LEV_FULL, H_LEV_CONE, H_REC_FULL, H_REC_CONE, H_MTASKS, H_OFF_LEV_FULL, H_OFF_LEV_CONE,
-    H_OFF_FF, H_OFF_PO, H_OFF_RAM, H_OFF_REC_FULL, H_OFF_REC_CONE, H_OFF_MT, H_OFF_PREDS,
-    H_OFF_REC_MT, H_REC_MT, H_TOTAL, H_WORDS = 32
-};
+using namespace gnplan;   // the program's header words
+
 constexpr uint32_t kMagic = 0x54474652u;  // 'RFGT'
 constexpr uint32_t kVersion = 1;
-constexpr uint32_t kDstMask = (1u << 29) - 1;
 
 #define GN_HIP(call)                                                                      \
     do {                                                                                  \
@@ -277,6 +274,16 @@ struct rf_gatenet {
     hipGraph_t bgraph[32] = {};
     hipGraphExec_t bexec[32] = {};
     uint32_t bnodes[32] = {};
+    // LDS form of the bit-plane mode: planned (or found not to fit, pb = 0),
+    // cycles run before; plane width in bytes, the plan's tables and rows, the
+    // workgroups' state between launches
+    bool planned = false;
+    uint64_t cycles = 0;
+    uint32_t pb = 0;
+    rf_gnl_params lp{};
+    uint32_t* lwords = nullptr;
+    uint2* lrows = nullptr;
+    uint32_t* limage = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
 };
 
@@ -543,6 +550,79 @@ int check_program(const uint32_t* h, size_t words) {
     return RF_OK;
 }
 
+// When the LDS form is planned: the plan of a netlist of R records takes about
+// 0.12 us per record on the host (60 ms for the 500,000-gate net5) and saves
+// about 90 us per cycle there (122 us level by level, 34 us in LDS), so it has
+// paid after R / 700 cycles; the handle plans once its runs reach R / 512.
+constexpr uint64_t kPlanRecords = 512;
+
+// Plan the LDS form and load its tables; leaves pb = 0 when the netlist does
+// not fit (its live planes exceed a workgroup's LDS even at 8 stimuli).
+int plan_lds(rf_gatenet* g) {
+    const uint32_t* h = H(g);
+    gnplan::Net net;
+    if (!h[H_PO] || !read_net(h, net)) return RF_OK;
+    gnplan::Planner pl(net, RF_GNL_THREADS / 64);
+    const uint32_t slots = pl.schedule();
+    // the widest planes that fit: a row costs the same for 8 stimuli as for 32
+    uint32_t pb = 0;
+    for (uint32_t b : {4u, 2u, 1u})
+        if (!pb && (uint64_t)slots * b + 4 <= RF_GNL_LDS) pb = b;
+    if (!pb) return RF_OK;
+    const gnplan::Plan p = pl.emit(pb);
+    GN_HIP(hipMalloc(&g->lwords, std::max<size_t>(4, p.words.size() * 4)));
+    GN_HIP(hipMemcpy(g->lwords, p.words.data(), p.words.size() * 4, hipMemcpyHostToDevice));
+    GN_HIP(hipMalloc(&g->lrows, p.rows.size() * 8));
+    GN_HIP(hipMemcpy(g->lrows, p.rows.data(), p.rows.size() * 8, hipMemcpyHostToDevice));
+    rf_gnl_params& q = g->lp;
+    q.words = g->lwords;
+    q.rows = g->lrows;
+    q.off_po = p.off_po;
+    q.off_ram = p.off_ram;
+    q.ram_words = p.ram_words;
+    q.n_pi = h[H_PI];
+    q.n_po = h[H_PO];
+    q.n_ram = p.n_ram_live;
+    q.n_rams = h[H_RAMS];
+    q.depth = h[H_DEPTH];
+    q.width = h[H_WIDTH];
+    q.abits = h[H_ABITS];
+    q.a0 = p.a0 * pb;
+    q.b0 = p.b0 * pb;
+    q.state_bytes = (p.nstate * pb + 3u) & ~3u;
+    q.lds_bytes = std::max((p.nslots * pb + 3u) & ~3u, q.state_bytes);
+    q.nlanes = g->nlanes;
+    q.M = g->M;
+    q.hash = g->hash;
+    q.budget = g->budget;
+    q.sid = g->sid;
+    g->pb = pb;
+    return RF_OK;
+}
+
+// The whole workload in the LDS form: launches of at most kLaunchCycles
+// cycles over the groups that still run (a prefix: lanes are sorted by
+// budget), each group leaving at its own longest budget.
+constexpr uint32_t kLaunchCycles = 16384;
+int run_lds(rf_gatenet* g, uint64_t seed, const std::vector<uint32_t>& lane_budget) {
+    rf_gnl_params q = g->lp;
+    const uint32_t W = 8 * g->pb;
+    const uint32_t ng = (g->nlanes + W - 1) / W;
+    const uint64_t last = (uint64_t)lane_budget[0] + 1;   // iterations of the longest group
+    if (lane_budget[0] >= kLaunchCycles && !g->limage)
+        GN_HIP(hipMalloc(&g->limage, (size_t)ng * q.state_bytes));
+    q.image = g->limage;
+    q.seed = seed;
+    for (uint64_t k = 0; k < last && lane_budget[0]; k += kLaunchCycles) {
+        q.k0 = (uint32_t)k;
+        q.k1 = (uint32_t)std::min<uint64_t>(k + kLaunchCycles, 0xffffffffull);
+        uint32_t n = 0;
+        while (n < ng && lane_budget[(size_t)n * W] >= k && lane_budget[(size_t)n * W]) ++n;
+        GN_HIP(rf_gnl_launch(q, g->pb, n, g->stream));
+    }
+    return RF_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -558,7 +638,7 @@ int rf_gn_destroy(rf_gatenet* g) {
         if (g->bexec[k]) (void)hipGraphExecDestroy(g->bexec[k]);
         if (g->bgraph[k]) (void)hipGraphDestroy(g->bgraph[k]);
     }
-    void* ps[] = {g->prog, g->P, g->X, g->M, g->hash, g->budget, g->ctl, g->sid};
+    void* ps[] = {g->prog, g->P, g->X, g->M, g->hash, g->budget, g->ctl, g->sid, g->lwords, g->lrows, g->limage};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     if (g->e0) (void)hipEventDestroy(g->e0);
@@ -607,6 +687,7 @@ uint32_t rf_gn_mtasks(const rf_gatenet* g) { return g ? H(g)[H_MTASKS] : 0; }
 
 uint32_t rf_gn_nodes_per_cycle(const rf_gatenet* g, uint32_t mode) {
     if (!g || mode > RF_GN_BITPLANE) return 0;
+    if (mode == RF_GN_BITPLANE && g->pb) return 0;   // no graph: whole runs are one kernel
     return mode == RF_GN_BITPLANE ? g->bnodes[g->lg] : g->nodes[mode];
 }
 
@@ -617,8 +698,18 @@ int rf_gn_run(rf_gatenet* g, uint32_t mode, uint64_t seed, const uint32_t* budge
     const uint32_t* h = H(g);
     if (mode == RF_GN_GRAPH && !h[H_MTASKS]) return rf_set_error(RF_E_STATE, "program has no mtask partition");
     const uint32_t ncyc = *std::max_element(budgets, budgets + g->nlanes);
+    // the LDS form's plan, once this handle's cycles pay for it
+    if (mode == RF_GN_BITPLANE && !g->planned) {
+        g->cycles += ncyc;
+        if (g->cycles * kPlanRecords >= h[H_REC_FULL]) {
+            g->planned = true;
+            int rc = plan_lds(g);
+            if (rc) return rc;
+        }
+    }
+    const bool in_lds = mode == RF_GN_BITPLANE && g->pb && ncyc < 0x80000000u;
     // state of this mode, allocated on first use
-    if (mode == RF_GN_BITPLANE && !g->P) {
+    if (mode == RF_GN_BITPLANE && !in_lds && !g->P) {
         const size_t bytes = ((size_t)h[H_NODES] << g->lg) * 8;
         GN_HIP(hipMalloc(&g->P, bytes));
     }
@@ -642,12 +733,12 @@ int rf_gn_run(rf_gatenet* g, uint32_t mode, uint64_t seed, const uint32_t* budge
                          [&](uint32_t x, uint32_t y) { return budgets[x] > budgets[y]; });
         lane_budget.resize(n);
         for (uint32_t l = 0; l < n; ++l) lane_budget[l] = budgets[lane_sid[l]];
-        const uint32_t ng = (n + 63) / 64;
+        const uint32_t ng = in_lds ? 0 : (n + 63) / 64;
         std::vector<uint32_t> gmax(ng, 0);
-        for (uint32_t l = 0; l < n; ++l) gmax[l / 64] = std::max(gmax[l / 64], lane_budget[l]);
-        le_of.resize(ncyc);
+        for (uint32_t l = 0; l < n && !in_lds; ++l) gmax[l / 64] = std::max(gmax[l / 64], lane_budget[l]);
+        le_of.resize(in_lds ? 0 : ncyc);
         uint32_t active = ng;
-        for (uint32_t c = 0; c < ncyc; ++c) {
+        for (uint32_t c = 0; c < ncyc && !in_lds; ++c) {
             while (active > 1 && gmax[active - 1] <= c) --active;
             uint32_t e = 0;
             while ((1u << e) < active) ++e;
@@ -659,7 +750,9 @@ int rf_gn_run(rf_gatenet* g, uint32_t mode, uint64_t seed, const uint32_t* budge
         }
     }
     // the reset state: zero nodes and RAMs, hash basis, cycle 0
-    if (mode == RF_GN_BITPLANE)
+    if (in_lds)
+        ;   // the kernel starts from zero planes
+    else if (mode == RF_GN_BITPLANE)
         GN_HIP(hipMemsetAsync(g->P, 0, ((size_t)h[H_NODES] << g->lg) * 8, g->stream));
     else
         GN_HIP(hipMemsetAsync(g->X, 0, (size_t)h[H_NODES] * g->npad, g->stream));
@@ -676,7 +769,11 @@ int rf_gn_run(rf_gatenet* g, uint32_t mode, uint64_t seed, const uint32_t* budge
                        g->ctl, seed);
     GN_HIP(hipGetLastError());
     GN_HIP(hipEventRecord(g->e0, g->stream));
-    for (uint32_t c = 0; c < ncyc; ++c)
+    if (in_lds) {
+        int rc = run_lds(g, seed, lane_budget);
+        if (rc) return rc;
+    }
+    for (uint32_t c = 0; c < ncyc && !in_lds; ++c)
         GN_HIP(hipGraphLaunch(mode == RF_GN_BITPLANE ? g->bexec[le_of[c]] : g->exec[mode], g->stream));
     GN_HIP(hipEventRecord(g->e1, g->stream));
     GN_HIP(hipEventSynchronize(g->e1));

@@ -1,0 +1,90 @@
+"""The LDS planner of the gate-net engine (csrc/rf_gnplan.h) on the CPU: a
+model of the kernel (gnplan_host.cpp) runs the planned wavefront programs and
+must hash as the C oracle does, over netlists with and without RAMs, ragged
+levels and outputs or flip-flops driven by inputs, flip-flops or RAM data;
+within a level no row may read what another writes."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+import oracle
+from rtlflow_amd import gatenet as gn
+from rtlflow_amd.designs.netlist import generate
+
+ROOT = Path(__file__).resolve().parent
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    so = tmp_path_factory.mktemp("gnplan") / "gnplan.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", str(ROOT.parent / "rtlflow_amd" / "csrc"),
+                    str(ROOT / "gnplan_host.cpp"), "-o", str(so)], check=True)
+    return C.CDLL(str(so))
+
+
+def plan_run(host, prog, waves, seed, budgets):
+    b = np.asarray(budgets, np.uint32)
+    out, info = np.zeros(len(b), np.uint64), np.zeros(5, np.uint32)
+    rc = host.gnplan_run(prog.ctypes.data_as(C.c_void_p), waves, C.c_uint64(seed), b.ctypes.data_as(C.c_void_p),
+                         len(b), out.ctypes.data_as(C.c_void_p), info.ctypes.data_as(C.c_void_p))
+    return rc, out, info
+
+
+NETS = [dict(n_gates=900, n_ff=90, n_pi=100, n_po=40, depth=9, n_rams=2, ram_depth=48, ram_width=20),
+        dict(n_gates=5000, n_ff=700, n_pi=64, n_po=64, depth=30),
+        dict(n_gates=40, n_ff=5, n_pi=3, n_po=2, depth=3),
+        dict(n_gates=3000, n_ff=300, n_pi=128, n_po=7, depth=6, n_rams=3, ram_depth=64, ram_width=64)]
+
+
+@pytest.mark.parametrize("k", range(len(NETS)))
+@pytest.mark.parametrize("waves", [1, 16])
+def test_planned_programs_hash_as_the_oracle(host, k, waves):
+    table = generate(seed=0x51A + k, **NETS[k])[1]
+    budgets = [7, 0, 1, 30]
+    prog = gn.program(table, threads=None)
+    rc, got, info = plan_run(host, prog, waves, 0xABCDEF, budgets)
+    assert rc == 0
+    want = oracle.netlist_run(table.to_bytes(), 0xABCDEF, len(budgets), budgets=budgets)
+    assert (got == want).all()
+    assert info[0] < table.first_gate + table.n_gates + 2 * table.n_pi
+
+
+def test_sources_at_outputs_flip_flops_and_ports(host):
+    """Outputs, D inputs and RAM ports that are inputs, flip-flops (a shift
+    chain among them) or RAM data, several flip-flops on one value, outputs
+    of equal gates."""
+    table = generate(seed=0x77, n_gates=300, n_ff=40, n_pi=20, n_po=10, depth=5, n_rams=1, ram_depth=16,
+                     ram_width=8)[1]
+    g0 = table.first_gate
+    ff = table.n_pi + np.arange(table.n_ff)
+    table.ff_d[1:8] = ff[0:7]                       # a shift chain
+    table.ff_d[8:12] = 3                            # an input, four times
+    table.ff_d[12] = table.n_pi + table.n_ff + 2    # RAM data
+    table.ff_d[13:17] = g0 + 17                     # one gate, four times
+    table.po[0:4] = [0, ff[7], table.n_pi + table.n_ff, g0 + 17]
+    table.ram_addr[0][:2] = [1, ff[3]]
+    table.ram_wdata[0][:3] = [2, ff[12], table.n_pi + table.n_ff + 5]
+    budgets = [25, 3, 40]
+    for waves in (1, 4):
+        rc, got, _ = plan_run(host, gn.program(table, threads=None), waves, 99, budgets)
+        assert rc == 0
+        assert (got == oracle.netlist_run(table.to_bytes(), 99, len(budgets), budgets=budgets)).all()
+
+
+def test_programs_out_of_level_order_are_not_planned(host):
+    """A cone that lacks a gate, or a record that reads its own level, keeps
+    the level-by-level form."""
+    table = generate(seed=5, n_gates=400, n_ff=30, n_pi=16, n_po=8, depth=6)[1]
+    prog = gn.program(table, threads=None)
+    n_cone, off = int(prog[14]), int(prog[22])
+    assert plan_run(host, prog, 4, 1, [2])[0] == 0
+    bad = prog.copy()
+    bad[off + 4 * (n_cone - 1)] ^= 1 << 29          # another operator in the cone
+    assert plan_run(host, bad, 4, 1, [2])[0] == 1
+    full = int(prog[21])
+    bad = prog.copy()
+    bad[full + 1] = bad[full + 4] & ((1 << 29) - 1)  # the first record reads the second's node
+    assert plan_run(host, bad, 4, 1, [2])[0] == 1

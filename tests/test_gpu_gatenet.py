@@ -50,6 +50,42 @@ def test_config5_full_size_bitplane_matches_oracle(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name,lanes,warm", [("net5", 200, 1000), ("net5_small", 1, 0), ("net5_small", 33, 12),
+                                             ("net5_small", 9000, 20)])
+def test_lds_form_matches_oracle(gpu, name, lanes, warm):
+    """After ``warm`` cycles the handle runs in LDS: ragged last workgroups,
+    budgets of 0, the same handle twice, and hashes equal to the level-by-level
+    form's (the first, short runs)."""
+    tb = registry.gatenet_table(name)
+    budgets = np.random.default_rng(lanes).integers(0, 40, size=lanes).astype(np.uint32)
+    budgets[0] = 40
+    print(f"gatenet lds {name} lanes={lanes}", flush=True)
+    with GateNet(registry.gatenet_program(name), lanes) as g:
+        first, _ = g.run(GateNet.BITPLANE, SEED, np.minimum(budgets, 2))
+        g.run(GateNet.BITPLANE, SEED, np.full(lanes, warm, np.uint32))
+        got, _ = g.run(GateNet.BITPLANE, SEED, budgets)
+        assert g.nodes_per_cycle(GateNet.BITPLANE) == 0
+        again, _ = g.run(GateNet.BITPLANE, SEED, np.minimum(budgets, 2))
+    assert (first == again).all()
+    k = min(lanes, 16 if name == "net5" else 512)
+    for s0 in {0, lanes - k}:
+        want = oracle.netlist_run(tb, SEED, k, stim0=s0, budgets=budgets[s0:s0 + k])
+        assert (got[s0:s0 + k] == want).all(), s0
+
+
+@pytest.mark.gpu
+def test_lds_form_across_launches(gpu):
+    """A budget past one launch's 16,384 cycles: the state goes on in the next
+    launch (a lane next to it stops before, another just at the boundary)."""
+    budgets = np.array([16390, 16383, 16384, 20, 0], np.uint32)
+    tb = registry.gatenet_table("net5_small")
+    print("gatenet lds net5_small two launches", flush=True)
+    with GateNet(registry.gatenet_program("net5_small"), len(budgets)) as g:
+        got, _ = g.run(GateNet.BITPLANE, SEED, budgets)
+    assert (got == oracle.netlist_run(tb, SEED, len(budgets), budgets=budgets)).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("schedule", ["heuristic", "learned"])
 def test_config5_full_size_graph_form_matches_oracle(gpu, schedule):
     if schedule not in registry.gatenet_meta("net5")["schedules"]:
