@@ -61,7 +61,8 @@ def build_runtime(force: bool = False) -> Path:
             CSRC / "rf_gnlds.hip"]
     deps = srcs + [INCLUDE / "rf_verilated.h", INCLUDE / "rf_design.h", INCLUDE / "rf_mlp.h",
                    INCLUDE / "rf_gatenet.h", CSRC / "rf_bitplane.h", CSRC / "rf_stim.h",
-                   CSRC / "rf_transpose.h", CSRC / "rf_gnlds.h", CSRC / "rf_gnplan.h"]
+                   CSRC / "rf_transpose.h", CSRC / "rf_gnlds.h", CSRC / "rf_gnplan.h",
+                   CSRC / "rf_bpplan.h"]
     if out.exists() and not force and all(out.stat().st_mtime >= p.stat().st_mtime for p in deps):
         return out
     BUILD.mkdir(parents=True, exist_ok=True)

@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "rf_design.h"
 
 #define RF_BP_DEFAULT_THREADS 512
@@ -25,13 +27,18 @@ enum { RF_BP_A0 = 0, RF_BP_M = 1, RF_BP_B = 2 };
 
 struct rf_bp_params {
     rf_args a;
-    // program M as rounds of one gate per thread, for the kernels that keep
-    // every thread's gate records in registers across cycles: round i covers
-    // the gate records [rb[i], re[i]) (uint2 index from ``prog``), thread t
-    // takes record rb[i] + t; bit i of ``bar``: a barrier follows.
+    // program M as rounds of wavefront rows (rf_bpplan.h), for the kernels
+    // that keep every thread's gate records in registers across cycles:
+    // ``plan`` holds the records [round][thread], then the classes at word
+    // off_cls; bit i of ``bar``: a barrier follows round i. nr = 0: program M
+    // is streamed level by level from ``prog``.
     uint32_t nr;
     uint64_t bar;
-    uint32_t rb[RF_BP_MAXR], re[RF_BP_MAXR];
+    const uint32_t* plan;
+    uint32_t off_cls;
+    // program M's commit pairs, hashed-output table and ports are read from
+    // ``tab``: the plan's words, or the blob (nr = 0)
+    const uint32_t* tab;
     const uint32_t* prog;     // device copy of the blob
     uint32_t nslots;
     uint32_t n_in, n_state, n_commit[2], n_hash, n_f;
@@ -66,13 +73,17 @@ struct rf_bp_params {
 };
 
 // Parse and check a blob (every slot index, level table and section size);
-// fills every field but ``a``, ``prog`` and the round table. Returns 0, or -1
+// fills every field but ``a``, ``prog``, ``tab`` and the plan's. Returns 0, or -1
 // with a reason in *why.
 int rf_bp_parse(const uint32_t* blob, uint64_t words, rf_bp_params* p, const char** why);
 
-// Fill the round table of program M for ``threads`` threads per
-// workgroup; nr = 0 when it needs more than RF_BP_MAXR rounds.
-void rf_bp_rounds(const uint32_t* blob, uint32_t threads, rf_bp_params* p);
+// Plan program M for ``threads`` threads per workgroup: the plan's words (for
+// p->plan and p->tab) and the fields that describe them. False (nr = 0, the
+// fields left) when it needs more rounds than the kernels hold in registers.
+bool rf_bp_plan(const uint32_t* blob, uint32_t threads, rf_bp_params* p, std::vector<uint32_t>* words);
+
+// The LDS layout behind the planes (tab_off, bal_off) from the table sizes.
+void rf_bp_layout(rf_bp_params* p);
 
 // Launch one kernel over ceil(nlanes / 64) workgroups (grp_n with group
 // rotation) of ``threads`` threads (128, 256, 512 or 1024).

@@ -12,10 +12,22 @@
 //   dst = s ? (x ^ ix) : (y ^ iy)        (a bit-select per 32-bit half)
 //
 // which covers AND, OR, XOR, NAND, NOR, XNOR, NOT and 2:1 MUX with the
-// inversions folded into ix / iy.
+// inversions folded into ix / iy. The per-cycle program M runs as rounds of
+// wavefront rows (rf_bpplan.h): 64 gates of one class, two or three operand
+// reads and no inversions.
+//
+// Bound (20,000-gate netlist, three workgroups per CU): LDS, busy 69 % of the
+// CU cycles (a 64-bit access of a wavefront takes 2.5 cycles to read and 6 to
+// write, and one more per extra slot in a bank pair), VALU issue 49 %, scalar
+// issue 32 %. As generic records (three reads and 12 VALU instructions a gate)
+// VALU issue was 69 % and LDS 64 %: 65,536 stimuli x 2,000 cycles 13.5 ms,
+// now 12.5 ms; 5,000 x 333 (one workgroup on a third of the CUs, bound by a
+// cycle's latency) 1.59 ms, now 1.41 ms.
 #include <algorithm>
+#include <utility>
 
 #include "rf_bitplane.h"
+#include "rf_bpplan.h"
 #include "rf_stim.h"
 #include "rf_transpose.h"
 
@@ -135,48 +147,6 @@ __device__ __forceinline__ void bp_gate_bytes(uint32_t dst, uint32_t s, uint32_t
     const uint32_t sl = (uint32_t)S, sh = (uint32_t)(S >> 32);
     *reinterpret_cast<lds_u64*>((size_t)dst) =
         ((uint64_t)((sh & xh) | (~sh & yh)) << 32) | (uint64_t)((sl & xl) | (~sl & yl));
-}
-
-// A register-resident byte-form record, decoded by an opaque instruction
-// sequence: the compiler can neither hoist the six decoded fields out of
-// the cycle loop (six registers per record instead of two) nor needs a copy
-// of the record to keep it intact. The empty record (x = 0xffffffff, no
-// valid destination offset 0xffff) is tested on the decoded field for the
-// same reason: a test of the record itself would be hoisted as a lane mask
-// per record.
-__device__ __forceinline__ void bp_gate_bytes_live(uint2 w) {
-    uint32_t dst, s, xs, ys, ix, iy;
-    asm volatile(
-        "v_and_b32 %0, 0xffff, %6\n\t"
-        "v_lshrrev_b32 %1, 16, %6\n\t"
-        "v_and_b32 %2, 0xfff8, %7\n\t"
-        "v_and_b32_sdwa %3, %7, %8 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:DWORD\n\t"
-        "v_bfe_i32 %4, %7, 0, 1\n\t"
-        "v_bfe_i32 %5, %7, 16, 1"
-        : "=&v"(dst), "=&v"(s), "=&v"(xs), "=&v"(ys), "=&v"(ix), "=&v"(iy)
-        : "v"(w.x), "v"(w.y), "s"(0xfff8u));
-    if (dst != 0xffffu) bp_gate_bytes(dst, s, xs, ys, ix, iy);
-}
-
-// The slot form's register-resident record, decoded the same way into LDS
-// byte offsets (the planes start at LDS address 0): dst and s are the two
-// halves of x, shifted; xs and ys drop the inversion flags (bits 15 and 31
-// of y). The empty record's destination half 0xffff becomes 0x7fff8, which
-// no slot has (at most 0x7fff slots).
-__device__ __forceinline__ void bp_gate_slots_live(uint2 w) {
-    uint32_t dst, s, xs, ys, ix, iy;
-    asm volatile(
-        "v_lshlrev_b32_sdwa %0, %8, %6 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0\n\t"
-        "v_lshlrev_b32_sdwa %1, %8, %6 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1\n\t"
-        "v_lshlrev_b32 %2, 3, %7\n\t"
-        "v_and_b32 %2, %9, %2\n\t"
-        "v_lshrrev_b32 %3, 13, %7\n\t"
-        "v_and_b32 %3, %9, %3\n\t"
-        "v_bfe_i32 %4, %7, 15, 1\n\t"
-        "v_ashrrev_i32 %5, 31, %7"
-        : "=&v"(dst), "=&v"(s), "=&v"(xs), "=&v"(ys), "=&v"(ix), "=&v"(iy)
-        : "v"(w.x), "v"(w.y), "s"(3u), "s"(0x3fff8u));
-    if (dst != 0x7fff8u) bp_gate_bytes(dst, s, xs, ys, ix, iy);
 }
 
 template <bool BA>
@@ -376,7 +346,7 @@ __device__ __forceinline__ void bp_mem_store(const rf_args& a, const uint32_t* m
 __device__ __forceinline__ void bp_mem_ports(uint64_t* L, const rf_bp_params& P, uint32_t which,
                                              uint32_t wave, uint32_t nw, uint32_t t, uint32_t lane,
                                              bool inb, bool act) {
-    const uint32_t* pp = P.prog + P.off_ports[which];
+    const uint32_t* pp = (which ? P.tab : P.prog) + P.off_ports[which];
     const uint32_t n = pp[1];
     const uint32_t* mt = P.prog + P.off_mem;
     pp += 2;
@@ -409,10 +379,11 @@ __device__ __forceinline__ void bp_mem_ports(uint64_t* L, const rf_bp_params& P,
 // its planes may change freely during the launch.
 template <int NT>
 __device__ __forceinline__ void bp_commit(uint64_t* L, const uint32_t* c, uint32_t n, uint32_t tid) {
-    for (uint32_t i = tid; i < n; i += NT) L[c[2 * i]] = L[c[2 * i + 1]];
+    for (uint32_t i = tid; i < n; i += NT) L[c[2 * i]] = bp_ref(L, c[2 * i + 1]);
 }
 
-// Commit pairs packed as state slot | next-state slot << 16, in LDS. With
+// Commit pairs packed as state slot | next-state slot << 16 | inverted << 31,
+// in LDS. With
 // more than two wavefronts, wavefronts 0 and 1 take no pairs: they start
 // their lane work (inputs, hash) at once, which runs beside the commit.
 template <int NT>
@@ -421,31 +392,114 @@ __device__ __forceinline__ void bp_commit_lds(uint64_t* L, const lds_u32* c, uin
     if (tid < SKIP) return;
     for (uint32_t i = tid - SKIP; i < n; i += NT - SKIP) {
         const uint32_t e = c[i];
-        L[e & 0xffffu] = L[e >> 16];
+        const uint64_t v = L[(e >> 16) & 0x7fffu];
+        L[e & 0xffffu] = (e >> 31) ? ~v : v;
     }
 }
 
-// Rounds [i0, i1) of the register-resident gate records, a barrier where
-// the round table says a level ends.
-template <int MAXR, bool BA>
-__device__ __forceinline__ void bp_rounds(uint64_t* L, const uint2 (&d)[MAXR], const rf_bp_params& P) {
-    // the round count and barrier mask pass an opaque step each cycle, so
-    // the per-round tests stay scalar compares here instead of precomputed
-    // lane masks (which outgrow the scalar registers and spill)
-    uint32_t nr = P.nr;
-    uint64_t bar = P.bar;
-    __asm__ volatile("" : "+s"(nr), "+s"(bar));
-#pragma unroll
-    for (int i = 0; i < MAXR; ++i) {
-        if (i < (int)nr) {
-            if constexpr (BA) {
-                bp_gate_bytes_live(d[i]);
-            } else {
-                bp_gate_slots_live(d[i]);
-            }
-            if ((bar >> i) & 1ull) __syncthreads();
-        }
-    }
+// One round of program M from a register-resident record: this wavefront's
+// row is of the class whose bits are bit I of c0..c2 (rf_bpplan.h: AND, ANDN,
+// NOR, XOR, MUX, MUXN, generic), if bit I of act is set; a workgroup barrier
+// follows where bit I of bar is set. Written as one block: the compiler turns
+// the class tree into predicated merges (18 scalar instructions a round where
+// this takes at most 11), and decodes the record here so that its fields
+// cannot be hoisted out of the cycle loop (up to six registers per record
+// instead of two). The reads of s and x, which every class has, go out before
+// the class is looked at. Registers: v64 destination, v65 s, v66 x, v67 y
+// addresses, v[68:69] s and the result, v[70:71] x, v[72:73] y, v74, v75 the
+// generic record's inversions.
+#define BP_ROW_TAIL(Y_DECODE, INV_DECODE)                                             \
+    "ds_read_b64 v[68:69], v65\n\t"                                                   \
+    "ds_read_b64 v[70:71], v66\n\t"                                                   \
+    "s_bitcmp1_b64 %[c2], %[i]\n\t"                                                   \
+    "s_cbranch_scc1 4f\n\t"                                                           \
+    "s_bitcmp1_b64 %[c1], %[i]\n\t"                                                   \
+    "s_cbranch_scc1 2f\n\t"                                                           \
+    "s_bitcmp1_b64 %[c0], %[i]\n\t"                                                   \
+    "s_waitcnt lgkmcnt(0)\n\t"                                                        \
+    "s_cbranch_scc1 1f\n\t"                                                           \
+    "v_and_b32 v68, v68, v70\n\t"                                                     \
+    "v_and_b32 v69, v69, v71\n\t"                                                     \
+    "s_branch 8f\n"                                                                   \
+    "1:\n\t"                                                                          \
+    "v_bitop3_b32 v68, v68, v70, v70 bitop3:0x30\n\t"                                 \
+    "v_bitop3_b32 v69, v69, v71, v71 bitop3:0x30\n\t"                                 \
+    "s_branch 8f\n"                                                                   \
+    "2:\n\t"                                                                          \
+    "s_bitcmp1_b64 %[c0], %[i]\n\t"                                                   \
+    "s_waitcnt lgkmcnt(0)\n\t"                                                        \
+    "s_cbranch_scc1 3f\n\t"                                                           \
+    "v_bitop3_b32 v68, v68, v70, v70 bitop3:0x03\n\t"                                 \
+    "v_bitop3_b32 v69, v69, v71, v71 bitop3:0x03\n\t"                                 \
+    "s_branch 8f\n"                                                                   \
+    "3:\n\t"                                                                          \
+    "v_xor_b32 v68, v68, v70\n\t"                                                     \
+    "v_xor_b32 v69, v69, v71\n\t"                                                     \
+    "s_branch 8f\n"                                                                   \
+    "4:\n\t" Y_DECODE                                                                 \
+    "ds_read_b64 v[72:73], v67\n\t"                                                   \
+    "s_bitcmp1_b64 %[c1], %[i]\n\t"                                                   \
+    "s_cbranch_scc1 6f\n\t"                                                           \
+    "s_bitcmp1_b64 %[c0], %[i]\n\t"                                                   \
+    "s_waitcnt lgkmcnt(0)\n\t"                                                        \
+    "s_cbranch_scc1 5f\n\t"                                                           \
+    "v_bitop3_b32 v68, v68, v70, v72 bitop3:0xca\n\t"                                 \
+    "v_bitop3_b32 v69, v69, v71, v73 bitop3:0xca\n\t"                                 \
+    "s_branch 8f\n"                                                                   \
+    "5:\n\t"                                                                          \
+    "v_bitop3_b32 v68, v68, v70, v72 bitop3:0x3a\n\t"                                 \
+    "v_bitop3_b32 v69, v69, v71, v73 bitop3:0x3a\n\t"                                 \
+    "s_branch 8f\n"                                                                   \
+    "6:\n\t" INV_DECODE                                                               \
+    "s_waitcnt lgkmcnt(0)\n\t"                                                        \
+    "v_xor_b32 v70, v70, v74\n\t"                                                     \
+    "v_xor_b32 v71, v71, v74\n\t"                                                     \
+    "v_xor_b32 v72, v72, v75\n\t"                                                     \
+    "v_xor_b32 v73, v73, v75\n\t"                                                     \
+    "v_bitop3_b32 v68, v68, v70, v72 bitop3:0xca\n\t"                                 \
+    "v_bitop3_b32 v69, v69, v71, v73 bitop3:0xca\n"                                   \
+    "8:\n\t"                                                                          \
+    "ds_write_b64 v64, v[68:69]\n"                                                    \
+    "9:\n\t"                                                                          \
+    "s_bitcmp1_b64 %[bar], %[i]\n\t"                                                  \
+    "s_cbranch_scc0 7f\n\t"                                                           \
+    "s_waitcnt lgkmcnt(0)\n\t"                                                        \
+    "s_barrier\n"                                                                     \
+    "7:\n"
+#define BP_ROW_ARGS                                                                                             \
+    :: [x] "v"(w.x), [y] "v"(w.y), [act] "s"(act), [c0] "s"(c0), [c1] "s"(c1), [c2] "s"(c2), [bar] "s"(bar),    \
+       [three] "s"(3u), [i] "n"(I)                                                                              \
+    : "v64", "v65", "v66", "v67", "v68", "v69", "v70", "v71", "v72", "v73", "v74", "v75", "scc", "memory"
+
+template <int I, bool BA>
+__device__ __forceinline__ void bp_round(uint2 w, uint64_t act, uint64_t c0, uint64_t c1, uint64_t c2, uint64_t bar) {
+    if constexpr (BA)
+        asm volatile("s_bitcmp1_b64 %[act], %[i]\n\t"
+                     "s_cbranch_scc0 9f\n\t"
+                     "v_lshrrev_b32 v65, 16, %[x]\n\t"
+                     "v_and_b32 v66, 0xfff8, %[y]\n\t"
+                     "v_and_b32 v64, 0xffff, %[x]\n\t"
+                     BP_ROW_TAIL("v_lshrrev_b32 v67, 16, %[y]\n\tv_and_b32 v67, 0xfff8, v67\n\t",
+                                 "v_bfe_i32 v74, %[y], 0, 1\n\tv_bfe_i32 v75, %[y], 16, 1\n\t")
+                     BP_ROW_ARGS);
+    else
+        asm volatile("s_bitcmp1_b64 %[act], %[i]\n\t"
+                     "s_cbranch_scc0 9f\n\t"
+                     "v_lshlrev_b32_sdwa v65, %[three], %[x] dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1\n\t"
+                     "v_lshlrev_b32 v66, 3, %[y]\n\t"
+                     "v_and_b32 v66, 0x3fff8, v66\n\t"
+                     "v_lshlrev_b32_sdwa v64, %[three], %[x] dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0\n\t"
+                     BP_ROW_TAIL("v_lshrrev_b32 v67, 13, %[y]\n\tv_and_b32 v67, 0x3fff8, v67\n\t",
+                                 "v_bfe_i32 v74, %[y], 15, 1\n\tv_ashrrev_i32 v75, 31, %[y]\n\t")
+                     BP_ROW_ARGS);
+}
+#undef BP_ROW_TAIL
+#undef BP_ROW_ARGS
+
+template <int MAXR, bool BA, int... I>
+__device__ __forceinline__ void bp_rounds(const uint2 (&d)[MAXR], const uint64_t (&m)[4], uint64_t bar,
+                                          std::integer_sequence<int, I...>) {
+    (bp_round<I, BA>(d[I], m[3], m[0], m[1], m[2], bar), ...);
 }
 
 // Workgroup of NT threads (NT >= 128) per 64 lanes. Lane t of the group is
@@ -534,10 +588,11 @@ rf_bp_kernel(rf_bp_params P) {
     const lds_u32* ti = th + P.hash_words;
     if (P.tab_off) {
         lds_u32* w = reinterpret_cast<lds_u32*>((size_t)P.tab_off);
-        const uint32_t* cm = prog + P.off_commit[1];
-        for (uint32_t i = tid; i < P.n_commit[1]; i += NT) w[i] = cm[2 * i] | (cm[2 * i + 1] << 16);
+        const uint32_t* ct = P.tab + P.off_commit[1];
+        for (uint32_t i = tid; i < P.n_commit[1]; i += NT)
+            w[i] = ct[2 * i] | (ct[2 * i + 1] << 16) | (ct[2 * i + 1] & 0x80000000u);
         w += P.n_commit[1];
-        const uint32_t* hp = prog + P.off_hash[0];
+        const uint32_t* hp = P.tab + P.off_hash[0];
         for (uint32_t i = tid; i < P.hash_words; i += NT) w[i] = hp[i];
         w += P.hash_words;
         for (uint32_t i = tid; i < 4u * P.n_in; i += NT) w[i] = in_tab[i];
@@ -551,16 +606,18 @@ rf_bp_kernel(rf_bp_params P) {
     }
     constexpr int MR = MAXR > 0 ? MAXR : 1;
     uint2 d[MR];
+    uint64_t cm[4] = {0, 0, 0, 0};
     if constexpr (MAXR > 0) {
-        const uint2* pg = reinterpret_cast<const uint2*>(prog);
 #pragma unroll
         for (int i = 0; i < MAXR; ++i) {
-            d[i] = make_uint2(0xffffffffu, 0u);
-            if (i < (int)P.nr) {
-                const uint32_t idx = P.rb[i] + tid;
-                if (idx < P.re[i]) d[i] = pg[idx];
-            }
+            d[i] = make_uint2(0u, 0u);
+            if (i < (int)P.nr) d[i] = reinterpret_cast<const uint2*>(P.plan)[(uint32_t)i * NT + tid];
         }
+        const uint32_t* pc = P.plan + P.off_cls + 8u * (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            cm[k] = (uint32_t)__builtin_amdgcn_readfirstlane((int)pc[2 * k]) |
+                    (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)pc[2 * k + 1]) << 32;
     }
     const uint32_t N = ngroup;
     if (N) {
@@ -586,18 +643,18 @@ rf_bp_kernel(rf_bp_params P) {
                 else __builtin_amdgcn_s_setprio(0);
             }
             if constexpr (MAXR > 0)
-                bp_rounds<MR, BA>(L, d, P);
+                bp_rounds<MR, BA>(d, cm, P.bar, std::make_integer_sequence<int, MR>());
             else
                 bp_phase<NT, BA>(L, lev[RF_BP_M], gates[RF_BP_M], P.nlev[RF_BP_M], tid);
             if (P.tab_off)
                 bp_commit_lds<NT>(L, tc, P.n_commit[1], tid);
             else
-                bp_commit<NT>(L, prog + P.off_commit[1], P.n_commit[1], tid);
+                bp_commit<NT>(L, P.tab + P.off_commit[1], P.n_commit[1], tid);
             if (P.n_mem) bp_mem_ports(L, P, 1, wave, NW, t, lane, inb, act);
             if (w1) {
                 const bool cap = IO && a.out.data && act && n < lim;
                 const uint64_t hn = P.tab_off ? bp_hash<IO>(L, th, P.n_hash, h, t, a, cap, sid, cyc + n)
-                                              : bp_hash<IO>(L, prog + P.off_hash[0], P.n_hash, h, t, a, cap, sid,
+                                              : bp_hash<IO>(L, P.tab + P.off_hash[0], P.n_hash, h, t, a, cap, sid,
                                                             cyc + n);
                 if (act && n < lim) h = hn;
             } else if (w0) {
@@ -724,6 +781,9 @@ static bool bp_check_refs(const uint32_t* refs, uint32_t width, uint32_t nslots)
         if ((refs[i] & 0x7fffffffu) >= nslots) return false;
     return true;
 }
+
+// Rounds of register-resident records the kernels of a workgroup size hold.
+static uint32_t bp_max_rounds(uint32_t threads) { return threads < 256 ? 0u : threads >= 1024 ? 40u : RF_BP_MAXR; }
 
 int rf_bp_parse(const uint32_t* b, uint64_t words, rf_bp_params* p, const char** why) {
 #define BP_FAIL(msg)   \
@@ -876,6 +936,12 @@ int rf_bp_parse(const uint32_t* b, uint64_t words, rf_bp_params* p, const char**
             const uint32_t* c = b + p->off_commit[which] + 2 * k;
             if (c[0] >= p->nslots || c[1] >= p->nslots) BP_FAIL("bit-plane commit slot out of range");
         }
+    rf_bp_layout(p);
+    return 0;
+#undef BP_FAIL
+}
+
+void rf_bp_layout(rf_bp_params* p) {
     // the per-cycle tables go to LDS after the planes when that costs no
     // workgroup per CU (160 KB of LDS per CU)
     const uint64_t planes = (uint64_t)p->nslots * 8u;
@@ -886,30 +952,46 @@ int rf_bp_parse(const uint32_t* b, uint64_t words, rf_bp_params* p, const char**
     const uint64_t used = planes + (p->tab_off ? tab : 0u);
     const uint64_t bal = (used + 7u) & ~7ull;
     p->bal_off = (bal + 8u <= cu - 64u && cu / planes == cu / (bal + 8u)) ? (uint32_t)bal : 0u;
-    return 0;
-#undef BP_FAIL
 }
 
-void rf_bp_rounds(const uint32_t* b, uint32_t threads, rf_bp_params* p) {
+bool rf_bp_plan(const uint32_t* b, uint32_t threads, rf_bp_params* p, std::vector<uint32_t>* words) {
+    bpplan::Source s{};
+    s.blob = b;
+    s.byte_form = p->byte_addr != 0;
+    s.nslots = p->nslots;
+    s.n_in = p->n_in;
+    s.off_in = p->off_in;
+    s.n_state = p->n_state;
+    s.off_state = p->off_state;
+    s.nlev = p->nlev[RF_BP_M];
+    s.off_lev = p->off_lev[RF_BP_M];
+    s.off_gates = p->off_gates[RF_BP_M];
+    s.n_commit = p->n_commit[1];
+    s.off_commit = p->off_commit[1];
+    s.n_hash = p->n_hash;
+    s.off_hash = p->off_hash[0];
+    s.off_ports = p->off_ports[1];
     p->nr = 0;
     p->bar = 0;
-    uint32_t r = 0;
-    const uint32_t* lv = b + p->off_lev[RF_BP_M];
-    const uint32_t g = p->off_gates[RF_BP_M] / 2;   // uint2 index of the first record
-    for (uint32_t l = 0; l < p->nlev[RF_BP_M]; ++l) {
-        const uint32_t lo = lv[l], hi = lv[l + 1];
-        for (uint32_t s = lo; s < hi; s += threads) {
-            if (r >= RF_BP_MAXR) {
-                p->bar = 0;
-                return;
-            }
-            p->rb[r] = g + s;
-            p->re[r] = g + hi;
-            if (s + threads >= hi) p->bar |= 1ull << r;
-            ++r;
-        }
+    const bpplan::Plan pl = bpplan::Planner(s, threads, bp_max_rounds(threads)).run();
+    if (!pl.ok) return false;
+    p->nr = pl.nr;
+    p->bar = pl.bar;
+    words->assign(pl.recs.begin(), pl.recs.end());
+    p->off_cls = (uint32_t)words->size();
+    for (uint64_t c : pl.cls) {
+        words->push_back((uint32_t)c);
+        words->push_back((uint32_t)(c >> 32));
     }
-    p->nr = r;
+    p->off_commit[1] = (uint32_t)words->size();
+    p->n_commit[1] = (uint32_t)pl.commit.size() / 2;
+    words->insert(words->end(), pl.commit.begin(), pl.commit.end());
+    p->off_hash[0] = (uint32_t)words->size();
+    words->insert(words->end(), pl.hash.begin(), pl.hash.end());
+    p->off_ports[1] = (uint32_t)words->size();
+    words->insert(words->end(), pl.ports.begin(), pl.ports.end());
+    rf_bp_layout(p);
+    return true;
 }
 
 static uint32_t bp_tab_words(const rf_bp_params& p) {

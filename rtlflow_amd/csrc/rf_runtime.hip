@@ -98,6 +98,8 @@ struct rf_model {
     rf_stats stats{};
     rf_args base{};
     uint32_t* bp_prog = nullptr;   // device copy of the bit-plane program
+    uint32_t* bp_plan = nullptr;   // the plan of its per-cycle program, made on first use
+    bool bp_planned = false;
     unsigned long long* bp_progress = nullptr;  // progress counter of a bit-plane launch
     int bp_per_cu[2] = {0, 0};     // bit-plane workgroups per CU (plain / stream kernel), 0 = not asked yet
     rf_bp_params bp{};
@@ -292,9 +294,22 @@ int load_bitplane(rf_model* m) {
     const size_t bytes = d->bitplane_words * 4;
     RF_HIP(hipMalloc(&m->bp_prog, bytes));
     RF_HIP(hipMemcpy(m->bp_prog, b, bytes, hipMemcpyHostToDevice));
-    m->bp.prog = m->bp_prog;
+    m->bp.prog = m->bp.tab = m->bp_prog;
     RF_HIP(hipMalloc(&m->bp_progress, sizeof(unsigned long long)));
     m->bp.progress = m->bp_progress;
+    return RF_OK;
+}
+
+// Plan the per-cycle program on the model's first bit-plane run.
+int plan_bitplane(rf_model* m) {
+    if (m->bp_planned) return RF_OK;
+    std::vector<uint32_t> words;
+    if (rf_bp_plan(m->d->bitplane, m->cfg.bitplane_threads, &m->bp, &words)) {
+        RF_HIP(hipMalloc(&m->bp_plan, words.size() * 4));
+        RF_HIP(hipMemcpy(m->bp_plan, words.data(), words.size() * 4, hipMemcpyHostToDevice));
+        m->bp.plan = m->bp.tab = m->bp_plan;
+    }
+    m->bp_planned = true;
     return RF_OK;
 }
 
@@ -653,7 +668,7 @@ int rf_destroy(rf_model* m) {
     for (int c = 0; c < 4; ++c)
         if (m->cls[c]) (void)hipFree(m->cls[c]);
     void* ps[] = {m->mem, m->change, m->done, m->hash, m->cyc, m->stim, m->flags,
-                  m->budget, m->order, m->out_hash, m->images, m->bp_prog, m->bp_progress};
+                  m->budget, m->order, m->out_hash, m->images, m->bp_prog, m->bp_plan, m->bp_progress};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     for (void* p : m->image_bufs)
@@ -894,6 +909,10 @@ int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
     if (rc) return rc;
     rc = do_init(m);
     if (rc) return rc;
+    if (mode == RF_MODE_BITPLANE) {
+        rc = plan_bitplane(m);
+        if (rc) return rc;
+    }
     hipEvent_t e0;
     if (mode == RF_MODE_GRAPH) {
         if (!n) return RF_OK;
@@ -926,7 +945,6 @@ int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
         uint32_t launches = 1;
         if (mode == RF_MODE_BITPLANE) {
             rf_bp_params p = m->bp;
-            rf_bp_rounds(m->d->bitplane, m->cfg.bitplane_threads, &p);
             p.a = args_for(m, RF_PHASE_EVAL);
             p.a.ncycles = chunk;
             // groups beyond what the GPU holds at once rotate through
@@ -1347,7 +1365,8 @@ int rf_submit_queue_static(rf_model* m, uint64_t seed, const uint32_t* budgets, 
 // whole queue's size, for the kernel's budget lookups).
 static int bitplane_rounds(rf_model* m, uint64_t seed, const uint32_t* budgets, const uint32_t* ord,
                            uint32_t n, uint32_t nstim) {
-    int rc = RF_OK;
+    int rc = plan_bitplane(m);
+    if (rc) return rc;
     const uint32_t nl = m->nlanes;
     std::vector<uint64_t> h(m->npad, 0xcbf29ce484222325ull);
     std::vector<uint32_t> sid(m->npad, 0);
@@ -1375,7 +1394,6 @@ static int bitplane_rounds(rf_model* m, uint64_t seed, const uint32_t* budgets, 
         RF_HIP(hipMemsetAsync(m->cyc, 0, m->npad * 4, m->stream));
         if (!ncyc) continue;
         rf_bp_params p = m->bp;
-        rf_bp_rounds(m->d->bitplane, m->cfg.bitplane_threads, &p);
         p.a = args_for(m, RF_PHASE_EVAL);
         p.a.seed = seed;
         p.a.ncycles = ncyc;
