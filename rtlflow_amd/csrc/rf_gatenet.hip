@@ -551,8 +551,8 @@ int check_program(const uint32_t* h, size_t words) {
 }
 
 // When the LDS form is planned: the plan of a netlist of R records takes about
-// 0.12 us per record on the host (60 ms for the 500,000-gate net5) and saves
-// about 90 us per cycle there (122 us level by level, 34 us in LDS), so it has
+// 0.13 us per record on the host (65 ms for the 500,000-gate net5) and saves
+// about 95 us per cycle there (122 us level by level, 26 us in LDS), so it has
 // paid after R / 700 cycles; the handle plans once its runs reach R / 512.
 constexpr uint64_t kPlanRecords = 512;
 
@@ -577,6 +577,7 @@ int plan_lds(rf_gatenet* g) {
     rf_gnl_params& q = g->lp;
     q.words = g->lwords;
     q.rows = g->lrows;
+    q.batch = p.batch;
     q.off_po = p.off_po;
     q.off_ram = p.off_ram;
     q.ram_words = p.ram_words;

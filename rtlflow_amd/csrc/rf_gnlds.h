@@ -10,7 +10,8 @@
 
 struct rf_gnl_params {
     const uint32_t* words;    // the plan's tables
-    const uint2* rows;        // its rows, 64 per wavefront row
+    const uint2* rows;        // its rows, by lines
+    uint32_t batch;           // wavefront rows of its batches
     uint32_t off_po, off_ram, ram_words;
     uint32_t n_pi, n_po, n_ram, n_rams, depth, width, abits;
     uint32_t a0, b0;          // LDS byte addresses of input sets A and B

@@ -5,12 +5,15 @@
 // pass over the program, a workgroup barrier per level.
 //
 // Bound (net5: 178,000 live gates, 155,000 rows, 124 KB of planes at 8 stimuli
-// per workgroup, one workgroup per CU): VALU issue and LDS, about half a CU's
-// rate each, plus the drain at 14 barriers per cycle: 34 us a cycle for 2,048
-// stimuli at once, against 122 us for 4,096 level by level through HBM, where
-// the 31 dependent launches of a cycle bounded it whatever the number of
-// stimuli. A workgroup's cycle costs the same for 8 stimuli as for 32, and the
-// longest budget bounds the run, so small workgroups lose nothing.
+// per workgroup, one workgroup per CU): LDS is busy 55 % of a cycle (half of
+// that bank conflicts), VALU issue 39 %, the vector cache 42 %; the rest is the
+// drain at 14 barriers: 26 us a cycle for 2,048 stimuli at once, against 122 us
+// for 4,096 level by level through HBM, where the 31 dependent launches of a
+// cycle bounded it whatever the number of stimuli. A workgroup's cycle costs
+// the same for 8 stimuli as for 32, and the longest budget bounds the run, so
+// small workgroups lose nothing. Batches of 2 or 6 wavefront rows instead of 4:
+// 32 and 27 us. Rows loaded 8 instead of 16 bytes a lane: 35 us (the vector
+// cache serves 4 lanes a cycle).
 #include "rf_gnlds.h"
 
 #include "rf_gnplan.h"
@@ -53,79 +56,98 @@ __device__ __forceinline__ uint32_t row_op(uint32_t a, uint32_t b, uint32_t y, i
 }
 
 // The values of N wavefront rows of a class, all operand reads first.
-template <uint32_t CLS, int N, typename T>
-__device__ __forceinline__ void row_values(const uint2 (&R)[4], uint32_t (&v)[N]) {
+template <uint32_t CLS, int N, typename T, int B>
+__device__ __forceinline__ void row_values(const uint2 (&R)[B], uint32_t (&v)[N]) {
     uint32_t a[N], b[N], c[N];
 #pragma unroll
     for (int u = 0; u < N; ++u) {
         a[u] = ld<T>(R[u].x & kMask);
-        b[u] = ld<T>(R[u].y >> 14);
-        if constexpr (CLS != gnplan::kSingle) c[u] = ld<T>(__builtin_amdgcn_alignbit(R[u].y, R[u].x, 18) & kMask);
+        if constexpr (CLS != gnplan::kCopy) b[u] = ld<T>(R[u].y >> 14);
+        if constexpr (CLS == gnplan::kPair || CLS == gnplan::kMux)
+            c[u] = ld<T>(__builtin_amdgcn_alignbit(R[u].y, R[u].x, 18) & kMask);
     }
     __builtin_amdgcn_sched_barrier(0);   // (the scheduler would wait for a row before the next one's reads)
 #pragma unroll
     for (int u = 0; u < N; ++u) {
         if constexpr (CLS == gnplan::kMux) v[u] = bitop3<0xca>(a[u], b[u], c[u]);
-        else v[u] = row_op(a[u], b[u], R[u].y, 4);
-        if constexpr (CLS == gnplan::kPair) v[u] = row_op(v[u], c[u], R[u].y, 7);
+        else if constexpr (CLS == gnplan::kSingle) v[u] = row_op(a[u], b[u], R[u].y, 4);
+        else if constexpr (CLS == gnplan::kPair) v[u] = row_op(row_op(a[u], b[u], R[u].y, 4), c[u], R[u].y, 7);
+        else if constexpr (CLS == gnplan::kOp) v[u] = a[u] & b[u];
+        else if constexpr (CLS == gnplan::kOp + 1) v[u] = a[u] | b[u];
+        else if constexpr (CLS == gnplan::kOp + 2) v[u] = a[u] ^ b[u];
+        else if constexpr (CLS == gnplan::kOp + 3) v[u] = ~(a[u] & b[u]);
+        else v[u] = a[u];
     }
 }
 
 // A batch of n rows of one class (at most kBatch wavefront rows, all their
 // operand reads before the first write: rows of a level read nothing that the
 // level writes). Rows past n read what their addresses name and are dropped.
-template <uint32_t CLS, typename T>
-__device__ __forceinline__ void batch_rows(const uint2 (&R)[4], uint32_t n, uint32_t dst, uint32_t t) {
+template <uint32_t CLS, typename T, int B>
+__device__ __forceinline__ void batch_rows(const uint2 (&R)[B], uint32_t n, uint32_t dst, uint32_t t) {
     const uint32_t d = dst + t * (uint32_t)sizeof(T);
-    if (n > 64) {
-        uint32_t v[4];
-        row_values<CLS, 4, T>(R, v);
-        st<T>(d, v[0]);
-        if (n == 256) {
+    const auto put = [&](int u, uint32_t v) {   // (a copy's destination is its own, in the b field)
+        st<T>(CLS == gnplan::kCopy ? R[u].y >> 14 : d + u * 64 * (uint32_t)sizeof(T), v);
+    };
+    if constexpr (B > 1) {
+        if (n > 64) {
+            uint32_t v[B];
+            row_values<CLS, B, T, B>(R, v);
+            put(0, v[0]);
+            if (n == 64 * B) {
 #pragma unroll
-            for (int u = 1; u < 4; ++u) st<T>(d + u * 64 * sizeof(T), v[u]);
-        } else {
+                for (int u = 1; u < B; ++u) put(u, v[u]);
+            } else {
 #pragma unroll
-            for (int u = 1; u < 4; ++u)
-                if (t + u * 64 < n) st<T>(d + u * 64 * sizeof(T), v[u]);
+                for (int u = 1; u < B; ++u)
+                    if (t + u * 64 < n) put(u, v[u]);
+            }
+            return;
         }
-    } else {
-        uint32_t v[1];
-        row_values<CLS, 1, T>(R, v);
-        if (t < n) st<T>(d, v[0]);
     }
+    uint32_t v[1];
+    row_values<CLS, 1, T, B>(R, v);
+    if (t < n) put(0, v[0]);
 }
 
-template <typename T>
-__device__ __forceinline__ void batch_run(const uint2 (&R)[4], uint32_t w, uint32_t dst, uint32_t t) {
-    const uint32_t n = (w >> 2) & 511u, cls = w & 3u;
+template <typename T, int B>
+__device__ __forceinline__ void batch_run(const uint2 (&R)[B], uint32_t w, uint32_t dst, uint32_t t) {
+    const uint32_t n = (w >> 3) & 511u, cls = w & 7u;
     if (n) {
-        if (cls == gnplan::kSingle) batch_rows<gnplan::kSingle, T>(R, n, dst, t);
-        else if (cls == gnplan::kPair) batch_rows<gnplan::kPair, T>(R, n, dst, t);
-        else batch_rows<gnplan::kMux, T>(R, n, dst, t);
-    }
-    if (w >> 31) __syncthreads();
-}
-
-// The input words of cycle ``cyc`` for the workgroup's W lanes into planes at
-// ``a0`` (one wavefront): thread t builds word t / W of lane t % W, so one
-// 64 x 64 transpose turns up to 64 / W words into planes.
-template <typename T>
-__device__ __forceinline__ void gen_inputs(const rf_gnl_params& p, uint64_t stim, uint32_t cyc, uint32_t t) {
-    constexpr uint32_t W = 8 * sizeof(T), J = 64 / W;
-    const uint32_t words = (p.n_pi + 63) / 64;
-    for (uint32_t j0 = 0; j0 < words; j0 += J) {
-        const uint32_t j = j0 + t / W;
-        const uint64_t w = j < words ? rf_stim(p.seed, stim, cyc, j) : 0ull;
-        const uint64_t col = bp_transpose64(w, t);
-        for (uint32_t k = 0; k < J && j0 + k < words; ++k) {
-            const uint32_t i = 64 * (j0 + k) + t;
-            if (i < p.n_pi) st<T>(p.a0 + i * sizeof(T), (uint32_t)(col >> (k * W)));
+        if (cls < gnplan::kOp) {
+            if (cls == gnplan::kSingle) batch_rows<gnplan::kSingle, T, B>(R, n, dst, t);
+            else if (cls == gnplan::kPair) batch_rows<gnplan::kPair, T, B>(R, n, dst, t);
+            else batch_rows<gnplan::kMux, T, B>(R, n, dst, t);
+        } else if (cls < gnplan::kOp + 2) {
+            if (cls == gnplan::kOp) batch_rows<gnplan::kOp, T, B>(R, n, dst, t);
+            else batch_rows<gnplan::kOp + 1, T, B>(R, n, dst, t);
+        } else {
+            if (cls == gnplan::kOp + 2) batch_rows<gnplan::kOp + 2, T, B>(R, n, dst, t);
+            else if (cls == gnplan::kOp + 3) batch_rows<gnplan::kOp + 3, T, B>(R, n, dst, t);
+            else batch_rows<gnplan::kCopy, T, B>(R, n, dst, t);
         }
     }
 }
 
+// The input words of cycle ``cyc`` for the workgroup's W lanes (one
+// wavefront): thread t builds word t / W of lane t % W, so one 64 x 64
+// transpose turns up to 64 / W words (at least the two an engine takes) into
+// planes: thread t's bits [k W, (k + 1) W) are the plane of input 64 k + t.
 template <typename T>
+__device__ __forceinline__ uint64_t input_words(const rf_gnl_params& p, uint64_t stim, uint32_t cyc, uint32_t t) {
+    constexpr uint32_t W = 8 * sizeof(T);
+    const uint32_t j = t / W;
+    return bp_transpose64(64u * j < p.n_pi ? rf_stim(p.seed, stim, cyc, j) : 0ull, t);
+}
+template <typename T>
+__device__ __forceinline__ void put_inputs(const rf_gnl_params& p, uint64_t col, uint32_t t) {
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k)
+        if (64 * k + t < p.n_pi) st<T>(p.a0 + (64 * k + t) * sizeof(T), (uint32_t)(col >> (k * 8 * sizeof(T))));
+}
+
+// B: wavefront rows of the plan's batches.
+template <typename T, int B>
 __global__ void __launch_bounds__(RF_GNL_THREADS) rf_gnl_kernel(rf_gnl_params p) {
     constexpr uint32_t W = 8 * sizeof(T);          // lanes of the workgroup
     constexpr uint32_t NW = RF_GNL_THREADS / 64;
@@ -143,7 +165,7 @@ __global__ void __launch_bounds__(RF_GNL_THREADS) rf_gnl_kernel(rf_gnl_params p)
     uint32_t* img = p.image + (size_t)blockIdx.x * (p.state_bytes / 4);
     for (uint32_t i = tid; i < p.state_bytes / 4; i += RF_GNL_THREADS) L[i] = p.k0 ? img[i] : 0u;
     __syncthreads();
-    if (wave == 0 && p.k0 == 0) gen_inputs<T>(p, stim, 0, t);
+    if (wave == 0 && p.k0 == 0) put_inputs<T>(p, input_words<T>(p, stim, 0, t), t);
     uint64_t h = 0;
     uint32_t bud = 0;
     if (wave == 1 && t < W && inb) {
@@ -151,52 +173,90 @@ __global__ void __launch_bounds__(RF_GNL_THREADS) rf_gnl_kernel(rf_gnl_params p)
         bud = p.budget[lane];
     }
     const uint32_t po = wave == 1 && t < p.n_po ? p.words[p.off_po + t] : 0u;
-    // this wavefront's program: batch words and row stream. A batch's words and
-    // rows are loaded three batches ahead (an L2 read takes about as long as
-    // two batches), as vector loads and always kBatch wavefront rows, so that
-    // the loads in flight are known without branches and complete in order
-    // (scalar loads would make every LDS wait a wait for them too).
+    // this wavefront's program: batch words and row stream. A batch's rows are
+    // loaded three batches ahead (an L2 read takes about as long as two
+    // batches), always the plan's B wavefront rows, so that the loads in flight
+    // are known without branches and complete in order (scalar loads would
+    // make every LDS wait a wait for them too). The words of kChunk batches
+    // come with one load, four lanes a batch: a load of one address by all
+    // lanes would cost the vector cache as much as 16 bytes for each.
+    constexpr uint32_t kLine = B > 1 ? 1024 : 512, kChunk = 15;
     const uint32_t nb = __builtin_amdgcn_readfirstlane(p.words[4 * wave + 1]);
-    const uint4* prog = reinterpret_cast<const uint4*>(p.words + __builtin_amdgcn_readfirstlane(p.words[4 * wave]));
-    const uint2* rows = p.rows + (size_t)__builtin_amdgcn_readfirstlane(p.words[4 * wave + 2]) * 64;
-    uint32_t zero;                // 0 the compiler does not know: keeps the batch words' loads vector loads
-    __asm__("v_mov_b32 %0, 0" : "=v"(zero));
-    uint4 D[3];
-    uint2 R[3][4];
-    const auto fetch = [&](uint4& d, uint2(&Q)[4], uint32_t j, uint32_t row) {
-        d = prog[j + zero];
+    const uint32_t* prog = p.words + __builtin_amdgcn_readfirstlane(p.words[4 * wave]);
+    const char* rows = reinterpret_cast<const char*>(p.rows) +
+                       (size_t)__builtin_amdgcn_readfirstlane(p.words[4 * wave + 2]) * kLine;
+    const uint32_t tl = t * (kLine / 64);
+    uint2 R0[B], R1[B], R2[B];
+    const auto fetch = [&](uint2(&Q)[B], uint32_t line) {
+        const char* base = rows + (size_t)line * kLine;
+        if constexpr (B == 1) {
+            Q[0] = *reinterpret_cast<const uint2*>(base + tl);
+        } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) Q[u] = rows[row + u * 64u + t];
+            for (int u = 0; u < B; u += 2) {
+                const uint4 q = *reinterpret_cast<const uint4*>(base + u / 2 * kLine + tl);
+                Q[u] = make_uint2(q.x, q.y);
+                Q[u + 1] = make_uint2(q.z, q.w);
+            }
+        }
     };
-#pragma unroll
-    for (int u = 0; u < 3; ++u) fetch(D[u], R[u], u, __builtin_amdgcn_readfirstlane(prog[u].w));
+    uint32_t ahead = prog[t];             // the next chunk's words
+    const auto word_of = [&](uint32_t v, uint32_t j) {
+        return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)j);
+    };
+    fetch(R0, word_of(ahead, 3));
+    fetch(R1, word_of(ahead, 7));
+    fetch(R2, word_of(ahead, 11));
+    // The lane work that waits for memory or for long chains runs beside the
+    // first levels of the next cycle: wavefront 0 builds the next inputs,
+    // wavefront 1 folds the last outputs into the hash, a RAM's wavefront
+    // waits for the word it read and writes its planes.
+    uint64_t col = 0, outs = 0, word = 0;
+    uint32_t rd = ~0u;                    // planes that ``word`` is for
+    const int nbytes = p.n_po <= 8 ? 1 : p.n_po <= 16 ? 2 : p.n_po <= 32 ? 4 : 8;
+    const auto put_word = [&]() {
+        const uint64_t c = bp_transpose64(word, t);
+        if (t < p.width) st<T>(rd + t * sizeof(T), (uint32_t)c);
+        rd = ~0u;
+    };
+    const auto fold = [&](uint32_t cyc) {
+        const uint64_t v = bp_transpose64(outs, t);
+        if (cyc < bud) h = rf_fnv_bytes(h, v, nbytes);
+    };
     __syncthreads();
     for (uint32_t k = p.k0; k < kend; ++k) {
-        for (uint32_t j = 0; j < nb; j += 3) {
-            const uint32_t jn = j + 3 < nb ? j + 3 : 0u;
-#pragma unroll
-            for (int u = 0; u < 3; ++u) {
-                const uint32_t w = __builtin_amdgcn_readfirstlane(D[u].x);
-                const uint32_t dst = __builtin_amdgcn_readfirstlane(D[u].y);
-                const uint32_t row = __builtin_amdgcn_readfirstlane(D[u].z);
-                batch_run<T>(R[u], w, dst, t);
-                fetch(D[u], R[u], jn + u, row);
+        uint32_t level = 0;
+        if (wave == 0) col = input_words<T>(p, stim, k + 1, t);
+        else if (wave == 1 && k > p.k0 && k > 1) fold(k - 2);
+        for (uint32_t c = 0; c < nb; c += kChunk) {
+            const uint32_t now = ahead;
+            ahead = prog[4 * (c + kChunk < nb ? c + kChunk : 0u) + t];
+            const uint32_t m = min(kChunk, nb - c);
+            for (uint32_t j = 0; j < m; j += 3) {
+                const auto step = [&](uint2(&Q)[B], uint32_t i) {
+                    const uint32_t w = word_of(now, 4 * i), line = word_of(now, 4 * i + 2);
+                    batch_run<T, B>(Q, w, word_of(now, 4 * i + 1), t);
+                    fetch(Q, line);
+                    if (w >> 31) {
+                        if (++level == gnplan::kRamLevels && rd != ~0u) put_word();
+                        __syncthreads();
+                    }
+                };
+                step(R0, j);
+                step(R1, j + 1);
+                step(R2, j + 2);
             }
         }
         // lane work after the last level, beside the other wavefronts' commit
         // rows (their destinations are flip-flops, which nothing here touches)
         if (wave == 0) {
             for (uint32_t i = t; i < p.n_pi; i += 64) st<T>(p.b0 + i * sizeof(T), ld<T>(p.a0 + i * sizeof(T)));
-            if (k + 1 < kend || p.k1 <= N) gen_inputs<T>(p, stim, k + 1, t);
+            put_inputs<T>(p, col, t);
         } else if (wave == 1) {
-            if (k) {
-                const uint64_t row = t < p.n_po ? (uint64_t)ld<T>(po) : 0ull;
-                const uint64_t v = bp_transpose64(row, t);
-                const int nb = p.n_po <= 8 ? 1 : p.n_po <= 16 ? 2 : p.n_po <= 32 ? 4 : 8;
-                if (k - 1 < bud) h = rf_fnv_bytes(h, v, nb);
-            }
+            outs = t < p.n_po ? (uint64_t)ld<T>(po) : 0ull;
         } else {
             for (uint32_t r = wave - 2; r < p.n_ram; r += NW - 2) {
+                if (rd != ~0u) put_word();     // more RAMs than wavefronts: all but the last at once
                 const uint32_t* rw = p.words + p.off_ram + r * p.ram_words;
                 const uint32_t ctl = t <= p.abits ? rw[2 + t] : 0u;
                 const uint32_t dat = t < p.width ? rw[2 + p.abits + 1 + t] : 0u;
@@ -205,27 +265,34 @@ __global__ void __launch_bounds__(RF_GNL_THREADS) rf_gnl_kernel(rf_gnl_params p)
                 const uint32_t addr = (uint32_t)(aw & ((1ull << p.abits) - 1ull));
                 const bool on = t < W && inb && addr < p.depth;
                 uint64_t* mem = p.M + ((size_t)lane * p.n_rams + rw[0]) * p.depth;
-                const uint64_t old = on ? mem[addr] : 0ull;
+                word = on ? mem[addr] : 0ull;
                 const uint64_t wmask = p.width >= 64 ? ~0ull : ((1ull << p.width) - 1ull);
                 if (on && ((aw >> p.abits) & 1ull)) mem[addr] = wd & wmask;
-                const uint64_t col = bp_transpose64(old, t);
-                if (t < p.width) st<T>(rw[1] + t * sizeof(T), (uint32_t)col);
+                rd = __builtin_amdgcn_readfirstlane(rw[1]);
             }
         }
         __syncthreads();
     }
+    if (wave == 1 && kend > 1) fold(kend - 2);
+    if (rd != ~0u) put_word();
+    __syncthreads();
     if (wave == 1 && t < W && inb) p.hash[lane] = h;
     if (kend <= N)     // more iterations to come in the next launch
         for (uint32_t i = tid; i < p.state_bytes / 4; i += RF_GNL_THREADS) img[i] = L[i];
 }
 
-template <typename T>
-hipError_t launch(const rf_gnl_params& p, uint32_t groups, hipStream_t stream) {
-    const void* fn = reinterpret_cast<const void*>(&rf_gnl_kernel<T>);
+template <typename T, int B>
+hipError_t launch_b(const rf_gnl_params& p, uint32_t groups, hipStream_t stream) {
+    const void* fn = reinterpret_cast<const void*>(&rf_gnl_kernel<T, B>);
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)RF_GNL_LDS);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((rf_gnl_kernel<T>), dim3(groups), dim3(RF_GNL_THREADS), p.lds_bytes, stream, p);
+    hipLaunchKernelGGL((rf_gnl_kernel<T, B>), dim3(groups), dim3(RF_GNL_THREADS), p.lds_bytes, stream, p);
     return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch(const rf_gnl_params& p, uint32_t groups, hipStream_t stream) {
+    return p.batch == 1 ? launch_b<T, 1>(p, groups, stream) : launch_b<T, gnplan::kBatch>(p, groups, stream);
 }
 
 }  // namespace

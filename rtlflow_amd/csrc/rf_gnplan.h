@@ -16,7 +16,9 @@
 //    three operands, so the value in between costs no LDS access).
 //  * Classes. Rows are single gates, pairs or multiplexers; 64 rows of one
 //    class form a wavefront row. A single's or pair's operators are bits of the
-//    row (classes per operator would leave most wavefront rows partly empty).
+//    row (classes per operator would leave most wavefront rows partly empty),
+//    but a level's single gates of one operator are a class of their own when
+//    they fill a batch: 3 VALU instructions a row instead of 8.
 //  * Batches. A wavefront takes up to four wavefront rows of one class at a
 //    time, so that their operand reads are in flight together; the batches of
 //    a level go to the least loaded wavefront.
@@ -28,8 +30,9 @@
 //    the last level.
 //  * Temporaries are reused: a batch's slots are free after the last level
 //    that reads one of them (rows of a class are sorted by that level).
-//  * Banks. LDS serves 32 lanes at a time over 64 banks of 4 bytes: the rows of
-//    a class whose slots die together are ordered so that each 32 of them read
+//  * Banks. LDS serves accesses of at most 4 bytes 32 lanes at a time over 32
+//    banks, in as many passes as the most dwords in one bank: the rows of a
+//    class whose slots die together are ordered so that each 32 of them read
 //    distinct banks as far as possible.
 #pragma once
 #include <stdint.h>
@@ -50,12 +53,17 @@ enum {
 constexpr uint32_t kDstMask = (1u << 29) - 1;   // of a record's first word; the type above it
 
 // Row classes: a single gate a k b, the pair (a k1 b) k2 c, the multiplexer
-// a ? b : c. Operators k: 0 AND, 1 OR, 2 XOR, 3 NAND.
-constexpr uint32_t kSingle = 0, kPair = 1, kMux = 2;
-inline uint32_t row_reads(uint32_t cls) { return cls == kSingle ? 2u : 3u; }
+// a ? b : c, single gates of one operator (kOp + k), the copy of a to address
+// b (commit rows). Operators k: 0 AND, 1 OR, 2 XOR, 3 NAND.
+constexpr uint32_t kSingle = 0, kPair = 1, kMux = 2, kOp = 3, kCopy = 7, kClasses = 8;
 // Cost of a wavefront row in VALU instructions plus LDS passes (its share of
 // the CU), for the balance between wavefronts.
-inline uint32_t row_cost(uint32_t cls) { return cls == kSingle ? 16u : cls == kPair ? 27u : 17u; }
+inline uint32_t row_cost(uint32_t cls) {
+    return cls == kSingle ? 16u : cls == kPair ? 27u : cls == kMux ? 17u : cls == kCopy ? 8u : 11u;
+}
+// What a wavefront does beside a cycle's first levels, in the same measure:
+// the next inputs and the hash (level 1), a RAM's read data (level kRamLevels).
+constexpr uint32_t kInputCost = 150, kHashCost = 200, kRamCost = 100;
 
 // A row: three operand byte addresses of at most 18 bits, a in bits 0..17, c
 // in 18..35, b in 46..63; operator masks of k1 in bits 36..38 and k2 in bits
@@ -67,11 +75,19 @@ inline uint64_t pack_row(uint32_t a, uint32_t b, uint32_t c, uint32_t k1, uint32
     return (uint64_t)a | ((uint64_t)c << 18) | ((uint64_t)b << 46) | (op_bits(k1) << 36) | (op_bits(k2) << 39);
 }
 
-// A batch of a wavefront's program, four words: class in bits 0..1, rows in
-// 2..10 (at most 256; 0: none), bit 31: a workgroup barrier follows; the first
-// destination's byte address; the first row (in the wavefront's row stream)
-// of the batch kUnroll places on, cyclically; its own first row.
-constexpr uint32_t kBatch = 4;     // wavefront rows
+// A batch of a wavefront's program, four words: class in bits 0..2, rows in
+// 3..11 (at most 64 times the plan's wavefront rows per batch; 0: none), bit
+// 31: a workgroup barrier follows; the first destination's byte address; the
+// position in the wavefront's row stream (in lines) of the batch kUnroll
+// places on, cyclically; its own position. A line is what 64 lanes load at
+// once: one wavefront row of 8 bytes a lane, or with batches of kBatch
+// wavefront rows two of them interleaved, 16 bytes a lane (the vector cache
+// serves 4 lanes a cycle whatever they load).
+// RAM data read at a cycle's edge reaches its planes within the next cycle's
+// first levels (the RAM's wavefronts write them before the barrier that ends
+// level kRamLevels): rows that read it come after.
+constexpr uint32_t kRamLevels = 1;
+constexpr uint32_t kBatch = 4;     // most wavefront rows of a batch
 constexpr uint32_t kUnroll = 3;    // a wavefront's batches are a multiple of this
 
 struct Gate {
@@ -167,13 +183,14 @@ struct Plan {
     uint32_t nslots = 0;          // plane slots of a workgroup
     uint32_t nstate = 0;          // the first of them: inputs, RAM data, flip-flops (kept between launches)
     uint32_t nwaves = 0;
+    uint32_t batch = 0;           // wavefront rows of a batch: kBatch, or 1 (small netlists)
     uint32_t n_ram_live = 0;
     uint32_t a0 = 0, b0 = 0;      // slots of input sets A and B (n_pi each)
     // device tables: words[4 * w] = {first batch word, batches (a
-    // multiple of kUnroll), first row / 64, 0} of wavefront w; words[off_po + k]: byte address of output k; words[off_ram + r * ram_words] = {RAM, byte address of its
+    // multiple of kUnroll), first line, 0} of wavefront w; words[off_po + k]: byte address of output k; words[off_ram + r * ram_words] = {RAM, byte address of its
     // read data, abits + 1 control addresses, width data addresses}
     std::vector<uint32_t> words;
-    std::vector<uint64_t> rows;   // 64 per wavefront row
+    std::vector<uint64_t> rows;   // 64 per wavefront row, by lines
     uint32_t off_po = 0, off_ram = 0, ram_words = 0;
     uint32_t wave_rows = 0, levels = 0;   // of one cycle
 };
@@ -297,7 +314,7 @@ private:
     std::vector<uint32_t> order_;             // rows in batch order
     std::vector<Batch> batches_;
     std::vector<uint32_t> slot_;              // per value
-    uint32_t nslots_ = 0, nstate_ = 0;
+    uint32_t nslots_ = 0, nstate_ = 0, batch_ = kBatch;
 };
 
 inline void Planner::find_live() {
@@ -484,13 +501,17 @@ inline void Planner::set_levels() {
     for (Row& r : rows_) {
         uint32_t l = 0;
         for (uint32_t k = 0; k < r.nrd; ++k) {
-            if (r.rd[k] < g0) continue;
+            if (r.rd[k] < g0) {
+                if (r.rd[k] >= src_rd()) l = std::max(l, kRamLevels);
+                continue;
+            }
             l = std::max(l, asap[r.rd[k] - g0]);
             readers[r.rd[k] - g0]++;
         }
         asap[r.val - g0] = r.level = l + 1;
         lmax_ = std::max(lmax_, r.level);
     }
+    if (std::count(ram_live_.begin(), ram_live_.end(), 1)) lmax_ = std::max(lmax_, kRamLevels);
     auto scan = [&]() {
         last_.assign(g0, 0);
         for (const Row& r : rows_)
@@ -529,10 +550,10 @@ inline void Planner::set_levels() {
         for (uint32_t f = v.ffs; f != kNone; f = next_ff_[f]) {
             if (f == pick) continue;
             Row c{};
-            c.cls = kSingle;
+            c.cls = kCopy;
             c.val = kNone;
-            c.nrd = 2;
-            c.rd[0] = c.rd[1] = rows_[i].val;
+            c.nrd = 1;
+            c.rd[0] = rows_[i].val;
             c.level = lc;
             c.inplace = true;
             c.ff = f;
@@ -545,20 +566,30 @@ inline void Planner::set_levels() {
 
 // Rows into batches: by level, class, destination kind and death.
 inline void Planner::cut() {
+    std::vector<uint32_t> ops((size_t)(lmax_ + 2) * 4, 0);
+    for (const Row& r : rows_)
+        if (r.cls == kSingle) ++ops[r.level * 4 + r.k1];
+    for (Row& r : rows_)
+        if (r.cls == kSingle && ops[r.level * 4 + r.k1] >= 64 * kBatch) r.cls = kOp + r.k1;
     // (a counting sort: level, class, in place, death)
     const uint32_t nd = lmax_ + 2;
-    const auto key = [&](const Row& r) { return ((r.level * 3 + r.cls) * 2 + (r.inplace ? 1u : 0u)) * nd + r.death; };
-    std::vector<uint32_t> start((size_t)(lmax_ + 2) * 6 * nd + 1, 0);
+    const auto key = [&](const Row& r) {
+        return ((r.level * kClasses + r.cls) * 2 + (r.inplace ? 1u : 0u)) * nd + r.death;
+    };
+    std::vector<uint32_t> start((size_t)(lmax_ + 2) * kClasses * 2 * nd + 1, 0);
     for (const Row& r : rows_) ++start[key(r) + 1];
     for (size_t k = 1; k < start.size(); ++k) start[k] += start[k - 1];
     order_.resize(rows_.size());
     for (uint32_t i = 0; i < rows_.size(); ++i) order_[start[key(rows_[i])]++] = i;
+    // batches of one wavefront row when the levels hold fewer than two per
+    // wavefront on average: every wavefront gets some, and loads no more
+    batch_ = rows_.size() < (size_t)(lmax_ + 1) * 128 * nw_ ? 1 : kBatch;
     for (size_t i = 0; i < order_.size();) {
         const uint32_t level = rows_[order_[i]].level;
         size_t e = i;
         while (e < order_.size() && rows_[order_[e]].level == level) ++e;
-        // small levels take smaller batches, so that every wavefront gets some
-        const uint32_t most = 64 * (uint32_t)std::min<size_t>(kBatch, std::max<size_t>(1, (e - i) / (128 * nw_)));
+        // small levels take smaller batches likewise
+        const uint32_t most = 64 * (uint32_t)std::min<size_t>(batch_, std::max<size_t>(1, (e - i) / (128 * nw_)));
         while (i < e) {
             const Row& r = rows_[order_[i]];
             Batch b{(uint32_t)i, 0, r.cls, level, 0, level, r.inplace};
@@ -602,16 +633,16 @@ inline void Planner::place(uint32_t pb) {
         for (const Block& b : ends[l - 1]) pool.give(b.at, b.n);
         for (; w < batches_.size() && batches_[w].level == l; ++w) {
             Batch& x = batches_[w];
-            if (x.inplace) continue;
+            if (x.inplace && x.cls != kCopy) continue;
             if (pb) {
+                const auto same = [&](const Batch& y) {
+                    return y.level == l && y.cls == x.cls && y.inplace == x.inplace && y.death == x.death;
+                };
                 uint32_t e = w + 1;
-                while (e < batches_.size() && batches_[e].level == l && batches_[e].cls == x.cls &&
-                       !batches_[e].inplace && batches_[e].death == x.death)
-                    ++e;
-                if (w == 0 || batches_[w - 1].level != l || batches_[w - 1].cls != x.cls ||
-                    batches_[w - 1].inplace || batches_[w - 1].death != x.death)
-                    spread_banks(&x, batches_.data() + e, pb);
+                while (e < batches_.size() && same(batches_[e])) ++e;
+                if (w == 0 || !same(batches_[w - 1])) spread_banks(&x, batches_.data() + e, pb);
             }
+            if (x.inplace) continue;
             x.base = pool.take(x.n);
             for (uint32_t k = 0; k < x.n; ++k) slot_[rows_[order_[x.first + k]].val] = x.base + k;
             ends[x.death].push_back({x.base, x.n});
@@ -620,48 +651,61 @@ inline void Planner::place(uint32_t pb) {
     nslots_ = pool.top();
 }
 
+// Dwords that 32 lanes' accesses of one operand name, by bank.
+struct Banks {
+    uint32_t dw[32][6];
+    uint8_t n[32];
+    uint8_t most;
+    void clear() {
+        std::fill(n, n + 32, 0);
+        most = 0;
+    }
+    bool has(uint32_t d) const {
+        for (uint32_t i = 0; i < n[d & 31]; ++i)
+            if (dw[d & 31][i] == d) return true;
+        return false;
+    }
+    // 256 for another pass, plus the dwords already in the bank
+    uint32_t cost(uint32_t d) const {
+        const uint32_t c = n[d & 31];
+        return !c || has(d) ? (c || most ? 0u : 1u) : c + (c == most ? 256u : 0u);
+    }
+    void put(uint32_t d) {
+        if (has(d)) return;
+        if (n[d & 31] < 6) dw[d & 31][n[d & 31]++] = d;
+        most = std::max(most, n[d & 31]);
+    }
+};
+
 // Order the rows of batches [b, e) (consecutive in order_) greedily: each next
-// row is the one of the first kWindow left whose operands meet the fewest
-// other dwords in their banks within the current 32 lanes. A half-wavefront
-// ends at a batch's 32nd, 64th ... row.
+// row is the one of the first kWindow left whose operands need the fewest
+// further passes of the current 32 lanes.
 inline void Planner::spread_banks(const Batch* b, const Batch* e, uint32_t pb) {
-    constexpr uint32_t kWindow = 64;
+    constexpr uint32_t kWindow = 128;
     std::vector<uint32_t> left;
     for (const Batch* x = b; x < e; ++x)
         left.insert(left.end(), order_.begin() + x->first, order_.begin() + x->first + x->n);
-    uint32_t dw[3][64][4];
-    uint8_t cnt[3][64];
+    Banks bk[3];
     size_t at = 0;   // left[at ..) are not placed
     for (const Batch* x = b; x < e; ++x)
         for (uint32_t k = 0; k < x->n; ++k) {
             if (k % 32 == 0)
-                for (auto& c : cnt) std::fill(c, c + 64, 0);
-            uint32_t best = 0, least = ~0u;
-            const size_t end = std::min(left.size(), at + kWindow);
+                for (Banks& c : bk) c.clear();
+            size_t best = at;
+            uint32_t least = ~0u;
+            const size_t end = k % 32 ? std::min(left.size(), at + kWindow) : at + 1;
             for (size_t i = at; i < end && least; ++i) {
                 const Row& r = rows_[left[i]];
                 uint32_t c = 0;
-                for (uint32_t j = 0; j < r.nrd; ++j) {
-                    const uint32_t d = slot_[r.rd[j]] * pb / 4, bank = d & 63;
-                    bool same = false;
-                    for (uint32_t q = 0; q < std::min<uint32_t>(cnt[j][bank], 4); ++q) same |= dw[j][bank][q] == d;
-                    if (!same) c += cnt[j][bank];
-                }
-                if (c < least) least = c, best = (uint32_t)i;
+                for (uint32_t j = 0; j < r.nrd; ++j) c += bk[j].cost(slot_[r.rd[j]] * pb / 4);
+                if (c < least) least = c, best = i;
             }
             const uint32_t row = left[best];
             left[best] = left[at];
             left[at++] = row;
             order_[x->first + k] = row;
             const Row& r = rows_[row];
-            for (uint32_t j = 0; j < r.nrd; ++j) {
-                const uint32_t d = slot_[r.rd[j]] * pb / 4, bank = d & 63;
-                bool same = false;
-                for (uint32_t q = 0; q < std::min<uint32_t>(cnt[j][bank], 4); ++q) same |= dw[j][bank][q] == d;
-                if (same) continue;
-                if (cnt[j][bank] < 4) dw[j][bank][cnt[j][bank]] = d;
-                if (cnt[j][bank] < 255) ++cnt[j][bank];
-            }
+            for (uint32_t j = 0; j < r.nrd; ++j) bk[j].put(slot_[r.rd[j]] * pb / 4);
         }
 }
 
@@ -670,6 +714,8 @@ inline Plan Planner::tables(uint32_t pb) const {
     p.nslots = nslots_;
     p.nstate = nstate_;
     p.nwaves = nw_;
+    p.batch = batch_;
+    const uint32_t per = batch_ == 1 ? 64 : 128;   // rows of a line
     p.a0 = 0;
     p.b0 = n_.n_pi;
     p.levels = lmax_ + 1;
@@ -685,6 +731,10 @@ inline Plan Planner::tables(uint32_t pb) const {
         std::stable_sort(ids.begin(), ids.end(), [&](uint32_t x, uint32_t y) { return cost(x) > cost(y); });
         const uint32_t w0 = l > lmax_ ? std::min(nw_ / 2, 2 + p.n_ram_live) : 0;
         std::vector<uint32_t> load(nw_, 0);
+        // (the lane work beside the first levels)
+        if (l == 1 && nw_ > 2) load[0] = kInputCost, load[1] = kHashCost;
+        if (l == kRamLevels)
+            for (uint32_t r = 0; r < p.n_ram_live && 2 + r < nw_; ++r) load[2 + r] = kRamCost;
         std::vector<std::vector<uint32_t>> mine(nw_);
         for (uint32_t i : ids) {
             const uint32_t k = (uint32_t)(std::min_element(load.begin() + w0, load.end()) - load.begin());
@@ -695,7 +745,7 @@ inline Plan Planner::tables(uint32_t pb) const {
             std::sort(mine[k].begin(), mine[k].end());
             for (uint32_t i : mine[k]) {
                 const Batch& x = batches_[i];
-                words[k].insert(words[k].end(), {x.cls | (x.n << 2), x.base * pb, 0u, 0u});
+                words[k].insert(words[k].end(), {x.cls | (x.n << 3), x.base * pb, 0u, 0u});
                 list[k].push_back(i);
                 p.wave_rows += (x.n + 63) / 64;
             }
@@ -708,27 +758,32 @@ inline Plan Planner::tables(uint32_t pb) const {
     for (uint32_t k = 0; k < nw_; ++k) {
         while (words[k].empty() || words[k].size() % (4 * kUnroll)) words[k].insert(words[k].end(), 4, 0u);
         const uint32_t nb = (uint32_t)words[k].size() / 4;
-        uint32_t row = 0;
+        uint32_t line = 0;
         for (uint32_t j = 0; j < nb; ++j) {
-            words[k][4 * j + 3] = row;
-            words[k][4 * ((j + nb - kUnroll) % nb) + 2] = row;
-            row += (((words[k][4 * j] >> 2) & 511u) + 63) / 64 * 64;
+            words[k][4 * j + 3] = line;
+            words[k][4 * ((j + nb - kUnroll) % nb) + 2] = line;
+            line += (((words[k][4 * j] >> 3) & 511u) + per - 1) / per;
         }
         p.words[4 * k] = (uint32_t)p.words.size();
         p.words[4 * k + 1] = nb;
         p.words.insert(p.words.end(), words[k].begin(), words[k].end());
-        p.words[4 * k + 2] = (uint32_t)(p.rows.size() / 64);
+        p.words[4 * k + 2] = (uint32_t)(p.rows.size() / per);
         for (uint32_t i : list[k]) {
             const Batch& x = batches_[i];
-            for (uint32_t t = 0; t < (x.n + 63) / 64 * 64; ++t) {
+            const size_t at = p.rows.size();
+            p.rows.resize(at + (x.n + per - 1) / per * per);
+            for (uint32_t t = 0; t < p.rows.size() - at; ++t) {
                 const Row& r = rows_[order_[x.first + std::min(t, x.n - 1)]];
+                const uint32_t b = r.cls == kCopy ? slot_[src_ff() + r.ff] : slot_[r.rd[1]];
                 const uint32_t c = r.nrd > 2 ? slot_[r.rd[2]] * pb : 0u;
-                p.rows.push_back(pack_row(slot_[r.rd[0]] * pb, slot_[r.rd[1]] * pb, c, r.k1, r.k2));
+                // row t of a line of two: lane t % 64, half t / 64
+                const uint32_t in = t % per, to = per == 64 ? in : 2 * (in % 64) + in / 64;
+                p.rows[at + t / per * per + to] = pack_row(slot_[r.rd[0]] * pb, b * pb, c, r.k1, r.k2);
             }
         }
     }
-    // a batch's loads cover kBatch wavefront rows whatever it holds
-    p.rows.resize(p.rows.size() + 64 * kBatch, 0);
+    // a batch's loads cover the most lines whatever it holds
+    p.rows.resize(p.rows.size() + 64 * batch_, 0);
     p.off_po = (uint32_t)p.words.size();
     for (uint32_t v : po_val_) p.words.push_back(slot_[v] * pb);
     p.off_ram = (uint32_t)p.words.size();
@@ -740,6 +795,7 @@ inline Plan Planner::tables(uint32_t pb) const {
         p.words.push_back(slot_[src_rd() + r * n_.width] * pb);
         for (uint32_t k = 0; k < pw; ++k) p.words.push_back(slot_[ram_val_[r * pw + k]] * pb);
     }
+    p.words.resize(p.words.size() + 64, 0);   // 64 lanes load batch words at once
     return p;
 }
 

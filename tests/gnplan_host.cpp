@@ -24,7 +24,7 @@ uint32_t op(uint32_t m, uint32_t a, uint32_t b) {   // operator masks p, q, n
 // info[0..4]: slots, state slots, levels, wavefront rows, rows evaluated.
 // Returns 0, 1 when the program is not planned, 2 when a level's rows read a
 // slot that the same level writes, 3 when the wavefronts' barriers differ, 4
-// when a batch's row position is wrong.
+// when a batch's row position is wrong, 5 when a class's operator is.
 extern "C" int gnplan_run(const uint32_t* h, uint32_t nwaves, uint64_t seed, const uint32_t* budgets, uint32_t n,
                           uint64_t* hashes, uint32_t* info) {
     Net net;
@@ -63,22 +63,32 @@ extern "C" int gnplan_run(const uint32_t* h, uint32_t nwaves, uint64_t seed, con
                         }
                         const uint32_t* d = &p.words[wt[0] + 4 * rj[w]++];
                         const uint32_t* ahead = &p.words[wt[0] + 4 * ((rj[w] - 1 + kUnroll) % wt[1])];
-                        if (d[2] != ahead[3] || (((d[0] >> 2) & 511) && d[3] != 64 * ri[w])) return 4;
-                        const uint32_t cls = d[0] & 3, n = (d[0] >> 2) & 511;
+                        if (d[2] != ahead[3] || (((d[0] >> 3) & 511) && d[3] != ri[w])) return 4;
+                        const uint32_t per = p.batch == 1 ? 64 : 128;
+                        if (((d[0] >> 3) & 511) > 64 * p.batch) return 4;
+                        const uint32_t cls = d[0] & 7, n = (d[0] >> 3) & 511;
                         bar = d[0] >> 31;
                         for (uint32_t i = 0; i < n; ++i) {
-                            const uint64_t row = p.rows[64 * (size_t)(wt[2] + ri[w]) + i];
+                            const uint32_t to = p.batch == 1 ? i : i / 128 * 128 + 2 * (i % 64) + i % 128 / 64;
+                            const uint64_t row = p.rows[per * (size_t)(wt[2] + ri[w]) + to];
                             const uint32_t a = row & 0x3ffff, c = (row >> 18) & 0x3ffff, b = row >> 46;
                             const uint32_t m = (row >> 36) & 63;
-                            read[a] = read[b] = 1;
-                            if (cls != kSingle) read[c] = 1;
+                            ++info[4];
+                            read[a] = 1;
+                            if (cls == kCopy) {
+                                L[b] = L[a];
+                                written[b] = 1;
+                                continue;
+                            }
+                            read[b] = 1;
+                            if (cls == kPair || cls == kMux) read[c] = 1;
                             uint32_t v = cls == kMux ? (L[a] ? L[b] : L[c]) : op(m & 7, L[a], L[b]);
+                            if (cls >= kOp && (m & 7) != op_bits(cls - kOp)) return 5;
                             if (cls == kPair) v = op(m >> 3, v, L[c]);
                             L[d[1] + i] = v & 1;
                             written[d[1] + i] = 1;
-                            ++info[4];
                         }
-                        ri[w] += (n + 63) / 64;
+                        ri[w] += (n + per - 1) / per;
                     }
                 }
                 for (uint32_t i = 0; i < p.nslots; ++i)

@@ -35,6 +35,7 @@ def plan_run(host, prog, waves, seed, budgets):
 
 NETS = [dict(n_gates=900, n_ff=90, n_pi=100, n_po=40, depth=9, n_rams=2, ram_depth=48, ram_width=20),
         dict(n_gates=5000, n_ff=700, n_pi=64, n_po=64, depth=30),
+        dict(n_gates=9000, n_ff=1500, n_pi=128, n_po=64, depth=8),
         dict(n_gates=40, n_ff=5, n_pi=3, n_po=2, depth=3),
         dict(n_gates=3000, n_ff=300, n_pi=128, n_po=7, depth=6, n_rams=3, ram_depth=64, ram_width=64)]
 
