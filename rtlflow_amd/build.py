@@ -86,8 +86,9 @@ def build_design(name: str, sources: Dict[str, str], manifest: dict, jobs: int =
         h.update(fn.encode())
         h.update(sources[fn].encode())
     h.update(" ".join(HIP_FLAGS).encode())
-    for hdr in ("rf_ops.h", "rf_stim.h"):
-        h.update((CSRC / hdr).read_bytes())
+    for hdr in ("rf_ops.h", "rf_stim.h", "rf_packed.h"):
+        if hdr != "rf_packed.h" or any(hdr in text for text in sources.values()):
+            h.update((CSRC / hdr).read_bytes())
     h.update((INCLUDE / "rf_design.h").read_bytes())
     key = h.hexdigest()[:16]
     d = design_dir(name, key)

@@ -12,6 +12,7 @@ import hashlib
 import json
 from typing import Callable, Dict, List, Optional, Set, Tuple
 
+from .emit_packed import packed_mtask
 from .emit_hip import ARR, CTY, Gen, cty, edge_cond, is_wide, lit
 from .instrcount import process_cost
 from .ir import CLASS_BYTES, Assign, Design, Ref, Var, words_of
@@ -1524,7 +1525,13 @@ def _emit_source(comp: Compiled) -> str:
         for b in emit_bodies(comp):
             parts.append(b)
             parts.append("")
+    # the design hash (checkpoints carry it) is of the per-lane kernels: a
+    # packed mtask kernel leaves the same state
+    packed: Dict[int, str] = {}
     for k in range(len(comp.mtasks)):
+        pk = packed_mtask(comp, k)
+        if pk:
+            packed[len(parts)] = pk
         parts.append(emit_mtask_kernel(comp, k))
         parts.append("")
     parts.append(emit_eval_end(comp))
@@ -1556,6 +1563,11 @@ def _emit_source(comp: Compiled) -> str:
         parts.append("")
     body = "\n".join(parts)
     h = int(hashlib.sha1(body.encode()).hexdigest()[:16], 16)
+    if packed:
+        for k, pk in packed.items():
+            parts[k] = pk
+        parts[parts.index('#include "rf_stim.h"')] += '\n#include "rf_packed.h"'
+        body = "\n".join(parts)
     parts = [body, emit_descriptor(comp, h)]
     return "\n".join(parts)
 
