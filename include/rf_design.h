@@ -23,7 +23,8 @@
 extern "C" {
 #endif
 
-#define RF_DESIGN_ABI 8
+/* 9 adds rf_design.help_threads and k_fused_help; the runtime takes 8 too. */
+#define RF_DESIGN_ABI 9
 
 /* storage classes (include/rf_heavy.h:11-17: CData/SData/IData/QData) */
 enum { RF_CLS_C = 0, RF_CLS_S = 1, RF_CLS_I = 2, RF_CLS_Q = 3 };
@@ -158,6 +159,10 @@ typedef struct rf_design {
      * set and no input stream or output capture is */
     const void* k_fused_mw;
     uint32_t mw_waves;
+    /* fused kernel with helper wavefronts: one workgroup of help_threads
+     * threads per 64 stimuli (0 / NULL when the design has none) */
+    uint32_t help_threads;
+    const void* k_fused_help;
 } rf_design;
 
 typedef const rf_design* (*rf_design_get_fn)(void);

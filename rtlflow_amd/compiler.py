@@ -12,6 +12,7 @@ import hashlib
 import json
 from typing import Callable, Dict, List, Optional, Set, Tuple
 
+from .emit_helped import emit_fused_help
 from .emit_packed import packed_mtask
 from .emit_hip import ARR, CTY, Gen, cty, edge_cond, is_wide, lit
 from .instrcount import process_cost
@@ -1525,8 +1526,8 @@ def _emit_source(comp: Compiled) -> str:
         for b in emit_bodies(comp):
             parts.append(b)
             parts.append("")
-    # the design hash (checkpoints carry it) is of the per-lane kernels: a
-    # packed mtask kernel leaves the same state
+    # the design hash (checkpoints carry it) is of the plain kernels: packed
+    # mtask kernels and the helped one leave the same state
     packed: Dict[int, str] = {}
     for k in range(len(comp.mtasks)):
         pk = packed_mtask(comp, k)
@@ -1566,13 +1567,17 @@ def _emit_source(comp: Compiled) -> str:
     if packed:
         for k, pk in packed.items():
             parts[k] = pk
-        parts[parts.index('#include "rf_stim.h"')] += '\n#include "rf_packed.h"'
+        if any("rf_pk_active" in pk for pk in packed.values()):
+            parts[parts.index('#include "rf_stim.h"')] += '\n#include "rf_packed.h"'
         body = "\n".join(parts)
-    parts = [body, emit_descriptor(comp, h)]
+    hk, ht = emit_fused_help(comp)
+    if hk:
+        body += "\n" + hk + "\n"
+    parts = [body, emit_descriptor(comp, h, ht)]
     return "\n".join(parts)
 
 
-def emit_descriptor(comp: Compiled, h: int) -> str:
+def emit_descriptor(comp: Compiled, h: int, help_threads: int = 0) -> str:
     d = comp.design
     man = comp.manifest()
     out = []
@@ -1643,7 +1648,8 @@ def emit_descriptor(comp: Compiled, h: int) -> str:
     else:
         out.append("    0, 0ull,")
     mw_w = mw_waves(comp)
-    out.append(f"    (const void*)&rf_k_fused_mw, {mw_w}u" if mw_w else "    0, 0u")
+    out.append(f"    (const void*)&rf_k_fused_mw, {mw_w}u," if mw_w else "    0, 0u,")
+    out.append(f"    {help_threads}u, (const void*)&rf_k_fused_help" if help_threads else "    0u, 0")
     out.append("};")
     # the only exported symbol: kernels stay library-local so several design
     # libraries can live in one process

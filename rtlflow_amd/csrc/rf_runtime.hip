@@ -540,7 +540,7 @@ uint64_t rf_lane_stride(const rf_model* m) { return m ? m->npad : 0; }
 int rf_create(const rf_design* d, uint32_t n_lanes, const rf_config* cfg, rf_model** out) {
     if (!d || !out) return fail(RF_E_ARG, "rf_create: null design or output pointer");
     *out = nullptr;
-    if (d->abi != RF_DESIGN_ABI)
+    if (d->abi != RF_DESIGN_ABI && d->abi != 8u)   // 8: no k_fused_help
         return fail(RF_E_DESIGN, "design ABI %u, runtime expects %u", d->abi, RF_DESIGN_ABI);
     if (n_lanes == 0) return fail(RF_E_ARG, "rf_create: n_lanes must be > 0");
     if (cfg && cfg->bitplane_threads &&
@@ -900,6 +900,15 @@ static std::vector<bp_window> bp_rotation(uint32_t G, uint32_t S, uint32_t n, bo
     return plan;
 }
 
+// The fused form with helper wavefronts: up to four groups of 64 stimuli per CU,
+// which its LDS holds at once (the register-file ALU, 4,000 cycles, 256 CUs: four
+// groups a CU 3.0 ms -> 1.68, one 2.9 -> 0.81). Above that the groups would run
+// in rounds; the plain kernel's one wavefront per group fills the SIMDs.
+static bool helped(const rf_model* m) {
+    return m->d->abi >= 9u && m->d->k_fused_help && !streams_set(m) &&
+           (m->nlanes + 63u) / 64u <= 4u * (uint32_t)std::max(1, m->ncu);
+}
+
 int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
     if (!m) return fail(RF_E_ARG, "null model");
     if (mode > RF_MODE_BITPLANE) return fail(RF_E_ARG, "unknown run mode %u", mode);
@@ -936,6 +945,10 @@ int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
                 // one workgroup of mw_waves wavefronts per 64 stimuli
                 void* params[] = {&a};
                 RF_HIP(hipLaunchKernel(m->d->k_fused_mw, dim3((m->nlanes + 63u) / 64u), dim3(64u * m->d->mw_waves),
+                                       params, 0, m->stream));
+            } else if (helped(m)) {
+                void* params[] = {&a};
+                RF_HIP(hipLaunchKernel(m->d->k_fused_help, dim3((m->nlanes + 63u) / 64u), dim3(m->d->help_threads),
                                        params, 0, m->stream));
             } else {
                 rc = launch(m, streams_set(m) ? m->d->k_fused_io : m->d->k_fused, a);

@@ -83,6 +83,8 @@ class Gen:
         # same clocked group); None = every NBA target
         self.nb_needed: Optional[Set[Var]] = None
         self.write_through = False
+        # if / case trees of cheap assignments as selects instead of branches
+        self.select_cases = False
         # small memories held in LDS by whole-cycle kernels: var -> array name
         # (element word k of this thread at name[k][threadIdx.x])
         self.lds: Dict[Var, str] = {}
@@ -233,7 +235,14 @@ class Gen:
         if isinstance(e, MemRd):
             m = e.var
             ix = self.idx_tmp(e.idx)
-            return f"({ix} < {m.depth}u ? ({cty(w)}){self.mem_elem(m, ix)} : ({cty(w)})0)"
+            rd = f"({ix} < {m.depth}u ? ({cty(w)}){self.mem_elem(m, ix)} : ({cty(w)})0)"
+            if self.select_cases:
+                # read whether an arm wants it or not: no branch between the
+                # reads of a cycle, so their latencies overlap
+                t = self.tmp("mr")
+                self.emit(f"const {cty(w)} {t} = {rd};")
+                return t
+            return rd
         if isinstance(e, Sel):
             a = e.a
             if is_wide(a.width):
@@ -593,6 +602,8 @@ class Gen:
         for s in ss:
             if isinstance(s, Assign):
                 self.assign(s)
+            elif self.select_cases and isinstance(s, (If, Case)) and 0 < self._flat_leaves([s]) <= 48:
+                self.flat([s], None)
             elif isinstance(s, If):
                 c = self.ex(s.cond)
                 saved = set(self.avail)
@@ -613,6 +624,99 @@ class Gen:
                 self.case(s)
             else:
                 raise CompileError(f"statement {s!r} not supported")
+
+    # ---- if / case trees as selects (select_cases)
+    def _flat_leaves(self, ss: List[Stmt]) -> int:
+        """Assignments of a tree that ``flat`` takes: whole narrow variables
+        from cheap expressions under cheap conditions; -1 where it does not."""
+        n = 0
+        for s in ss:
+            if isinstance(s, Assign):
+                v = s.lhs.var
+                if not s.lhs.whole or v.is_mem or v.width > 32 or v in self.packed or \
+                        not (v in self.avail or v in self.nb) or not self._cheap(s.rhs):
+                    return -1
+                n += 1
+            elif isinstance(s, If):
+                if not self._cheap(s.cond):
+                    return -1
+                for x in (s.then, s.els or []):
+                    k = self._flat_leaves(x)
+                    if k < 0:
+                        return -1
+                    n += k
+            elif isinstance(s, Case):
+                if not self._cheap(s.expr) or any(lab is None for lab, _ in s.items[:-1]):
+                    return -1
+                for _, x in s.items:
+                    k = self._flat_leaves(x)
+                    if k < 0:
+                        return -1
+                    n += k
+            else:
+                return -1
+        return n
+
+    def _cheap(self, e: Expr) -> bool:
+        """Narrow, a handful of instructions; a memory read is one (guarded)."""
+        if e.width > 32:
+            return False
+        if isinstance(e, Const):
+            return True
+        if isinstance(e, Ref):
+            return not e.var.is_mem
+        if isinstance(e, MemRd):
+            return not is_wide(e.var.width) and self._cheap(e.idx)
+        if isinstance(e, Sel):
+            return isinstance(e.lsb, int) and self._cheap(e.a)
+        if isinstance(e, Cond):
+            return self._cheap(e.c) and self._cheap(e.a) and self._cheap(e.b)
+        if isinstance(e, Concat):
+            return all(self._cheap(x) for x in e.parts)
+        if isinstance(e, Op):
+            return e.op not in ("divu", "modu", "divs", "mods", "pow") and all(self._cheap(x) for x in e.args)
+        return False
+
+    def flat(self, ss: List[Stmt], pred: Optional[str]):
+        """Every arm is computed, every assignment takes its value where the
+        arm's condition ``pred`` holds."""
+        for s in ss:
+            if isinstance(s, Assign):
+                v = s.lhs.var
+                t = self.tmp("fv")
+                self.emit(f"const {cty(v.width)} {t} = {self.ex(s.rhs)};")
+                if v in self.nb:
+                    dst = self.target(v)
+                    self.emit(f"{dst} = {pred} ? {t} : {dst};")
+                else:
+                    self.emit(self.set(v, f"{pred} ? {t} : {self.get(v)}"))
+                    self.dirty.add(v)
+                    self._write_through(v)
+            elif isinstance(s, If):
+                c = self.tmp("fc")
+                self.emit(f"const bool {c} = ({self.ex(s.cond)}) != 0;")
+                for x, neg in ((s.then, ""), (s.els or [], "!")):
+                    if x:
+                        q = self.tmp("fp")
+                        self.emit(f"const bool {q} = {pred + ' & ' if pred else ''}{neg}{c};")
+                        self.flat(x, q)
+            else:
+                w = s.expr.width
+                sel = self.tmp("cs")
+                self.emit(f"const {cty(w)} {sel} = {self.ex(s.expr)};")
+                left = pred or "true"      # no item has matched yet
+                for labels, x in s.items:
+                    if labels is None:
+                        self.flat(x, left)
+                        break
+                    conds = [f"({sel} == {lit(val, w)})" if care == mask(w) else
+                             f"((({sel} ^ {lit(val, w)}) & {lit(care, w)}) == 0)" for val, care in labels]
+                    m, q, r = self.tmp("fm"), self.tmp("fp"), self.tmp("fr")
+                    self.emit(f"const bool {m} = {' | '.join(conds)};")
+                    self.emit(f"const bool {q} = {left} & {m};")
+                    self.emit(f"const bool {r} = {left} & !{m};")
+                    self.flat(x, q)
+                    left = r
 
     def case(self, s: Case):
         w = s.expr.width
