@@ -1075,6 +1075,20 @@ def plan_packing(comp: Compiled, gen: Gen, carried: Set[Var]):
                        "registers": (nxt + 31) // 32}
 
 
+# The batched kernel's straight form emits a cycle twice (a stimulus's first one
+# apart). Up to this many estimated instructions of a cycle: above are the
+# systolic array and the netlists (11,000 up), plain expressions without arms to
+# take out, whose kernels would compile twice as long. Batched runs of 700
+# stimuli over 300 lanes, plain -> straight: register-file ALU 1.24 -> 0.71 ms,
+# RV32I 3.57 -> 3.39 (1.3 times over long programs), a small netlist 3.50 ->
+# 2.51, random word-level designs 4.3 -> 2.5 to 14.6 -> 10.8. And up to this many
+# calls of the wide-word helpers, each a loop over words unrolled in place: 430
+# gain 1.35 times; with 1,100 the kernel grew from 14 to 41 KB and lost (2.0 ->
+# 5.0 ms), on instruction fetch.
+STRAIGHT_OPS = 4000
+STRAIGHT_WIDE = 600
+
+
 def _fused_locals(comp: Compiled) -> Set[Var]:
     sch = comp.sch
     loc = _vertex_vars(comp, list(range(len(sch.vertices))))
@@ -1527,7 +1541,8 @@ def _emit_source(comp: Compiled) -> str:
             parts.append(b)
             parts.append("")
     # the design hash (checkpoints carry it) is of the plain kernels: packed
-    # mtask kernels and the helped one leave the same state
+    # mtask kernels, straight batched ones and the helped one leave the same
+    # state
     packed: Dict[int, str] = {}
     for k in range(len(comp.mtasks)):
         pk = packed_mtask(comp, k)
@@ -1552,6 +1567,10 @@ def _emit_source(comp: Compiled) -> str:
         for io in (False, True):
             parts.append(emit_fused(comp, io))
             parts.append("")
+            if not comp.host and not comp.sch.change_vars and 2 * sum(comp.vcost) <= STRAIGHT_OPS:
+                straight = emit_persistent(comp, io, straight=True)
+                if straight.count("rfw_") <= STRAIGHT_WIDE:
+                    packed[len(parts)] = straight
             parts.append(emit_persistent(comp, io))
             parts.append("")
         mw, _ = emit_fused_mw(comp)
