@@ -37,6 +37,12 @@ from .layout import class_of
 # 60 and 40 / 120 is the same at 16,384, 4,096 and 300 lanes.
 CHUNK = 12
 KEEP = 60
+# Longer mtasks keep the per-lane kernel: hipcc's time for one straight kernel
+# with two instantiations grows faster than its length (a 50,000-gate design
+# with 16 of its 44 mtasks above this, up to 960: 381 s per-lane, 662 s all
+# packed), and a finer partition of such a design (its learned one has 253 at
+# most) has them packed.
+STMTS = 500
 CTY = {"C": "uint8_t", "S": "uint16_t", "I": "uint32_t", "Q": "uint64_t"}
 ARR = {"C": "sC", "S": "sS", "I": "sI", "Q": "sQ"}
 
@@ -307,6 +313,8 @@ def packed_mtask(comp, k: int) -> Optional[str]:
         return None
     try:
         g = _Gen(comp, k)
+        if len(g.stmts) > STMTS:
+            return None
         body = g.body()
     except Unpackable:
         return None
