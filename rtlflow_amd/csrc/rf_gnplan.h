@@ -571,16 +571,21 @@ inline void Planner::cut() {
         if (r.cls == kSingle) ++ops[r.level * 4 + r.k1];
     for (Row& r : rows_)
         if (r.cls == kSingle && ops[r.level * 4 + r.k1] >= 64 * kBatch) r.cls = kOp + r.k1;
-    // (a counting sort: level, class, in place, death)
-    const uint32_t nd = lmax_ + 2;
-    const auto key = [&](const Row& r) {
-        return ((r.level * kClasses + r.cls) * 2 + (r.inplace ? 1u : 0u)) * nd + r.death;
+    // (two stable counting sorts, by death, then by level, class and in place:
+    // their tables grow with the depth, not with its square, and hold any depth)
+    const auto sort_by = [&](const std::vector<uint32_t>& in, size_t keys, const auto& key) {
+        std::vector<uint32_t> start(keys + 1, 0), out(in.size());
+        for (uint32_t i : in) ++start[key(rows_[i]) + 1];
+        for (size_t k = 1; k < start.size(); ++k) start[k] += start[k - 1];
+        for (uint32_t i : in) out[start[key(rows_[i])]++] = i;
+        return out;
     };
-    std::vector<uint32_t> start((size_t)(lmax_ + 2) * kClasses * 2 * nd + 1, 0);
-    for (const Row& r : rows_) ++start[key(r) + 1];
-    for (size_t k = 1; k < start.size(); ++k) start[k] += start[k - 1];
     order_.resize(rows_.size());
-    for (uint32_t i = 0; i < rows_.size(); ++i) order_[start[key(rows_[i])]++] = i;
+    for (uint32_t i = 0; i < rows_.size(); ++i) order_[i] = i;
+    order_ = sort_by(order_, lmax_ + 2, [](const Row& r) { return (size_t)r.death; });
+    order_ = sort_by(order_, (size_t)(lmax_ + 2) * kClasses * 2, [](const Row& r) {
+        return ((size_t)r.level * kClasses + r.cls) * 2 + (r.inplace ? 1u : 0u);
+    });
     // batches of one wavefront row when the levels hold fewer than two per
     // wavefront on average: every wavefront gets some, and loads no more
     batch_ = rows_.size() < (size_t)(lmax_ + 1) * 128 * nw_ ? 1 : kBatch;

@@ -4,6 +4,7 @@ must hash as the C oracle does, over netlists with and without RAMs, ragged
 levels and outputs or flip-flops driven by inputs, flip-flops or RAM data;
 within a level no row may read what another writes."""
 import ctypes as C
+import resource
 import subprocess
 from pathlib import Path
 
@@ -12,7 +13,7 @@ import pytest
 
 import oracle
 from rtlflow_amd import gatenet as gn
-from rtlflow_amd.designs.netlist import generate
+from rtlflow_amd.designs.netlist import MUX, GateTable, generate
 
 ROOT = Path(__file__).resolve().parent
 
@@ -89,3 +90,27 @@ def test_programs_out_of_level_order_are_not_planned(host):
     bad = prog.copy()
     bad[full + 1] = bad[full + 4] & ((1 << 29) - 1)  # the first record reads the second's node
     assert plan_run(host, bad, 4, 1, [2])[0] == 1
+
+
+def test_deep_chain_plans_in_memory_linear_in_its_depth(host, monkeypatch):
+    """20,000 levels of one multiplexer each: the plan's tables grow with the
+    depth, not with its square (a key of level and death in 32 bits would wrap
+    from 16,384 levels on)."""
+    n, n_pi = 20000, 8
+    rng = np.random.default_rng(9)
+    first = n_pi + 1
+    gin = np.zeros((n, 3), np.uint32)
+    gin[:, 0] = rng.integers(0, n_pi, n)
+    gin[:, 1] = np.arange(first - 1, first - 1 + n)     # the gate before (first: the flip-flop)
+    gin[:, 2] = rng.integers(0, first, n)
+    swap = rng.random(n) < 0.5
+    gin[swap, 1], gin[swap, 2] = gin[swap, 2], gin[swap, 1].copy()
+    table = GateTable(n_pi, 1, 0, np.full(n, MUX, np.uint8), gin, np.array([first + n // 2], np.uint32),
+                      np.array([first + n - 1, first + n - 2], np.uint32))
+    monkeypatch.setattr(gn, "gate_levels", lambda t: np.arange(1, n + 1, dtype=np.int32))
+    budgets = [3, 1]
+    before = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+    rc, got, info = plan_run(host, gn.program(table, threads=None), 16, 0x77, budgets)
+    assert rc == 0 and info[2] == n + 1
+    assert resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before < 1 << 20    # KiB
+    assert (got == oracle.netlist_run(table.to_bytes(), 0x77, len(budgets), budgets=budgets)).all()
