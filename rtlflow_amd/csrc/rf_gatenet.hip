@@ -556,24 +556,28 @@ int check_program(const uint32_t* h, size_t words) {
 // paid after R / 700 cycles; the handle plans once its runs reach R / 512.
 constexpr uint64_t kPlanRecords = 512;
 
-// Plan the LDS form and load its tables; leaves pb = 0 when the netlist does
-// not fit (its live planes exceed a workgroup's LDS even at 8 stimuli).
-int plan_lds(rf_gatenet* g) {
+// Plan the LDS form and load its tables. Leaves pb = 0 where that is not
+// possible (plan_program, or no device memory for the tables): the handle then
+// goes on level by level.
+void plan_lds(rf_gatenet* g) {
     const uint32_t* h = H(g);
-    gnplan::Net net;
-    if (!h[H_PO] || !read_net(h, net)) return RF_OK;
-    gnplan::Planner pl(net, RF_GNL_THREADS / 64);
-    const uint32_t slots = pl.schedule();
-    // the widest planes that fit: a row costs the same for 8 stimuli as for 32
-    uint32_t pb = 0;
-    for (uint32_t b : {4u, 2u, 1u})
-        if (!pb && (uint64_t)slots * b + 4 <= RF_GNL_LDS) pb = b;
-    if (!pb) return RF_OK;
-    const gnplan::Plan p = pl.emit(pb);
-    GN_HIP(hipMalloc(&g->lwords, std::max<size_t>(4, p.words.size() * 4)));
-    GN_HIP(hipMemcpy(g->lwords, p.words.data(), p.words.size() * 4, hipMemcpyHostToDevice));
-    GN_HIP(hipMalloc(&g->lrows, p.rows.size() * 8));
-    GN_HIP(hipMemcpy(g->lrows, p.rows.data(), p.rows.size() * 8, hipMemcpyHostToDevice));
+    gnplan::Plan p;
+    const uint32_t pb = gnplan::plan_program(h, RF_GNL_THREADS / 64, RF_GNL_LDS, &p);
+    if (!pb) return;
+    const auto load = [](auto** dev, const auto& host) {
+        const size_t bytes = host.size() * sizeof(host[0]);
+        hipError_t e = hipMalloc(dev, bytes);
+        if (e == hipSuccess) e = hipMemcpy(*dev, host.data(), bytes, hipMemcpyHostToDevice);
+        return e == hipSuccess;
+    };
+    if (!load(&g->lwords, p.words) || !load(&g->lrows, p.rows)) {
+        (void)hipGetLastError();
+        if (g->lwords) (void)hipFree(g->lwords);
+        if (g->lrows) (void)hipFree(g->lrows);
+        g->lwords = nullptr;
+        g->lrows = nullptr;
+        return;
+    }
     rf_gnl_params& q = g->lp;
     q.words = g->lwords;
     q.rows = g->lrows;
@@ -598,20 +602,30 @@ int plan_lds(rf_gatenet* g) {
     q.budget = g->budget;
     q.sid = g->sid;
     g->pb = pb;
-    return RF_OK;
 }
 
 // The whole workload in the LDS form: launches of at most kLaunchCycles
 // cycles over the groups that still run (a prefix: lanes are sorted by
 // budget), each group leaving at its own longest budget.
 constexpr uint32_t kLaunchCycles = 16384;
+
+// Whether a run of ``ncyc`` cycles goes there: planned, and device memory for
+// the workgroups' state between launches where there is more than one.
+bool runs_in_lds(rf_gatenet* g, uint32_t ncyc) {
+    if (!g->pb || ncyc >= 0x80000000u) return false;
+    if (ncyc < kLaunchCycles || g->limage) return true;
+    const uint32_t W = 8 * g->pb;
+    if (hipMalloc(&g->limage, (size_t)((g->nlanes + W - 1) / W) * g->lp.state_bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    g->limage = nullptr;
+    return false;
+}
+
 int run_lds(rf_gatenet* g, uint64_t seed, const std::vector<uint32_t>& lane_budget) {
     rf_gnl_params q = g->lp;
     const uint32_t W = 8 * g->pb;
     const uint32_t ng = (g->nlanes + W - 1) / W;
     const uint64_t last = (uint64_t)lane_budget[0] + 1;   // iterations of the longest group
-    if (lane_budget[0] >= kLaunchCycles && !g->limage)
-        GN_HIP(hipMalloc(&g->limage, (size_t)ng * q.state_bytes));
     q.image = g->limage;
     q.seed = seed;
     for (uint64_t k = 0; k < last && lane_budget[0]; k += kLaunchCycles) {
@@ -704,11 +718,10 @@ int rf_gn_run(rf_gatenet* g, uint32_t mode, uint64_t seed, const uint32_t* budge
         g->cycles += ncyc;
         if (g->cycles * kPlanRecords >= h[H_REC_FULL]) {
             g->planned = true;
-            int rc = plan_lds(g);
-            if (rc) return rc;
+            plan_lds(g);
         }
     }
-    const bool in_lds = mode == RF_GN_BITPLANE && g->pb && ncyc < 0x80000000u;
+    const bool in_lds = mode == RF_GN_BITPLANE && runs_in_lds(g, ncyc);
     // state of this mode, allocated on first use
     if (mode == RF_GN_BITPLANE && !in_lds && !g->P) {
         const size_t bytes = ((size_t)h[H_NODES] << g->lg) * 8;

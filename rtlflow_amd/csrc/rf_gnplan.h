@@ -38,6 +38,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <exception>
 #include <map>
 #include <vector>
 
@@ -802,6 +803,28 @@ inline Plan Planner::tables(uint32_t pb) const {
     }
     p.words.resize(p.words.size() + 64, 0);   // 64 lanes load batch words at once
     return p;
+}
+
+// The plan of a checked program for workgroups of ``nwaves`` wavefronts and
+// ``lds_bytes`` of LDS: its plane width in bytes, or 0 when the program runs
+// level by level -- no outputs, not a plain levelised netlist, live planes
+// beyond the LDS even at 8 stimuli, or no host memory to plan it in (the
+// callers are C entry points, which no exception may leave).
+inline uint32_t plan_program(const uint32_t* h, uint32_t nwaves, uint64_t lds_bytes, Plan* out) noexcept {
+    try {
+        Net net;
+        if (!h[H_PO] || !read_net(h, net)) return 0;
+        Planner pl(net, nwaves);
+        const uint64_t slots = pl.schedule();
+        // the widest planes that fit: a row costs the same for 8 stimuli as for 32
+        for (uint32_t pb : {4u, 2u, 1u})
+            if (slots * pb + 4 <= lds_bytes) {
+                *out = pl.emit(pb);
+                return pb;
+            }
+    } catch (const std::exception&) {
+    }
+    return 0;
 }
 
 }  // namespace gnplan

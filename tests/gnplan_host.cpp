@@ -1,10 +1,23 @@
 // CPU model of the gate-net engine's LDS kernel: plans a program blob with
 // rf_gnplan.h and runs the wavefront programs over byte planes, one stimulus
 // per call. Built by tests/test_gnplan.py with the host compiler.
+#include <cstdlib>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "rf_gnplan.h"
+
+// Allocations left before one fails (negative: none does). Linked
+// -Bsymbolic, so only this file's allocations come here.
+static long g_left = -1;
+void* operator new(size_t n) {
+    if (g_left >= 0 && g_left-- == 0) throw std::bad_alloc();
+    if (void* p = malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 using namespace gnplan;
 
@@ -20,6 +33,18 @@ uint32_t op(uint32_t m, uint32_t a, uint32_t b) {   // operator masks p, q, n
     return (m & 2 ? t ^ b : t & b) ^ (m >> 2);
 }
 }  // namespace
+
+// The plane width that plan_program chooses when its allocation ``left`` fails;
+// *used: the allocations it made.
+extern "C" uint32_t gnplan_width(const uint32_t* h, uint32_t nwaves, uint64_t lds_bytes, long left, long* used) {
+    Plan p;
+    g_left = left >= 0 ? left : 1l << 40;
+    const long l0 = g_left;
+    const uint32_t pb = plan_program(h, nwaves, lds_bytes, &p);
+    *used = l0 - g_left;
+    g_left = -1;
+    return pb;
+}
 
 // info[0..4]: slots, state slots, levels, wavefront rows, rows evaluated.
 // Returns 0, 1 when the program is not planned, 2 when a level's rows read a

@@ -21,7 +21,8 @@ ROOT = Path(__file__).resolve().parent
 @pytest.fixture(scope="module")
 def host(tmp_path_factory):
     so = tmp_path_factory.mktemp("gnplan") / "gnplan.so"
-    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", str(ROOT.parent / "rtlflow_amd" / "csrc"),
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wl,-Bsymbolic", "-I",
+                    str(ROOT.parent / "rtlflow_amd" / "csrc"),
                     str(ROOT / "gnplan_host.cpp"), "-o", str(so)], check=True)
     return C.CDLL(str(so))
 
@@ -114,3 +115,21 @@ def test_deep_chain_plans_in_memory_linear_in_its_depth(host, monkeypatch):
     assert rc == 0 and info[2] == n + 1
     assert resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before < 1 << 20    # KiB
     assert (got == oracle.netlist_run(table.to_bytes(), 0x77, len(budgets), budgets=budgets)).all()
+
+
+def test_plan_without_memory_is_no_plan(host):
+    """Whichever allocation of the planner fails, the program is not planned
+    (it runs level by level) and no exception leaves the planner."""
+    prog = gn.program(generate(seed=0x51A, **NETS[0])[1], threads=None)
+    used = C.c_long(0)
+
+    def width(left, lds=160 * 1024):
+        return host.gnplan_width(prog.ctypes.data_as(C.c_void_p), 16, C.c_uint64(lds), C.c_long(left), C.byref(used))
+
+    assert width(-1) == 4
+    total = used.value
+    assert total > 100
+    for left in sorted({0, 1, 2, *range(0, total, max(1, total // 97)), total - 1}):
+        assert width(left) == 0, left
+    assert width(total) == 4
+    assert width(-1, lds=256) == 0
