@@ -23,8 +23,9 @@
 extern "C" {
 #endif
 
-/* 9 adds rf_design.help_threads and k_fused_help; the runtime takes 8 too. */
-#define RF_DESIGN_ABI 9
+/* 9 adds rf_design.help_threads and k_fused_help, 10 the bit-plane plans; the
+ * runtime takes 8 and 9 too. */
+#define RF_DESIGN_ABI 10
 
 /* storage classes (include/rf_heavy.h:11-17: CData/SData/IData/QData) */
 enum { RF_CLS_C = 0, RF_CLS_S = 1, RF_CLS_I = 2, RF_CLS_Q = 3 };
@@ -115,6 +116,12 @@ typedef struct rf_args {
     rf_stream out;       /* output capture (data null: none) */
 } rf_args;
 
+typedef struct rf_bp_plan_words {
+    uint32_t threads;
+    uint64_t n;
+    const uint32_t* words;
+} rf_bp_plan_words;
+
 typedef struct rf_design {
     uint32_t abi;              /* RF_DESIGN_ABI */
     uint32_t block;            /* threads per block the kernels assume */
@@ -163,6 +170,10 @@ typedef struct rf_design {
      * threads per 64 stimuli (0 / NULL when the design has none) */
     uint32_t help_threads;
     const void* k_fused_help;
+    /* plans of the bit-plane program's per-cycle part, one per workgroup size
+     * that has one (csrc/rf_bpplan.h) */
+    const rf_bp_plan_words* bp_plans;
+    uint32_t n_bp_plans;
 } rf_design;
 
 typedef const rf_design* (*rf_design_get_fn)(void);

@@ -1164,6 +1164,32 @@ def encode(prog: Program) -> List[int]:
     return out
 
 
+PLAN_THREADS = (256, 512, 1024)   # workgroup sizes whose kernels keep records in registers
+_PLAN_SECTIONS = ("in", "state", "levM", "gatesM", "commitM", "hashM", "portsM")
+
+
+def plan(blob: Sequence[int], threads: int) -> Optional[List[int]]:
+    """u32 words of the plan of the per-cycle program for workgroups of
+    ``threads`` threads (csrc/rf_bpplan.h), or None where the runtime runs the
+    program's own records."""
+    import ctypes as C
+
+    import numpy as np
+
+    from .build import build_planner
+    lib = C.CDLL(str(build_planner()))
+    lib.rf_bpplan_make.restype = C.c_uint64
+    b = np.asarray(blob, np.uint32)
+    sec = sections(blob)
+    s = np.array([sec[k] for k in _PLAN_SECTIONS], np.uint32)
+    # at most 48 rounds of two words a thread, the classes, the blob's tables
+    out = np.zeros(2 * 48 * threads + 4096 + 2 * len(b), np.uint32)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    n = int(lib.rf_bpplan_make(p(b), p(s), threads, p(out), C.c_uint64(len(out))))
+    assert n <= len(out), (n, len(out))
+    return out[:n].tolist() if n else None
+
+
 def sections(blob: Sequence[int]) -> Dict[str, object]:
     """Word offsets of every section of an encoded program (the runtime
     computes the same offsets from the header)."""

@@ -73,6 +73,18 @@ def build_runtime(force: bool = False) -> Path:
     return out
 
 
+def build_planner() -> Path:
+    """The bit-plane planner as a host library (used while designs compile)."""
+    out = BUILD / "host" / "librf_bpplan.so"
+    deps = [CSRC / "rf_bpplan.cpp", CSRC / "rf_bpplan.h"]
+    if not out.exists() or any(out.stat().st_mtime < p.stat().st_mtime for p in deps):
+        out.parent.mkdir(parents=True, exist_ok=True)
+        tmp = out.with_suffix(f".so.tmp{os.getpid():x}")
+        _run(["g++", "-O3", "-std=c++17", "-shared", "-fPIC", str(deps[0]), "-o", str(tmp)])
+        os.replace(tmp, out)
+    return out
+
+
 def design_dir(name: str, key: str) -> Path:
     return BUILD / "designs" / f"{name}_{key}"
 

@@ -1645,6 +1645,20 @@ def emit_descriptor(comp: Compiled, h: int, help_threads: int = 0) -> str:
         for i in range(0, len(blob), 16):
             out.append("    " + ", ".join(f"{x}u" for x in blob[i:i + 16]) + ",")
         out.append("};")
+    plans = []
+    if comp.bitplane_blob and not comp.host:
+        from . import bitplane as bp
+        for th in bp.PLAN_THREADS:
+            words = bp.plan(comp.bitplane_blob, th)
+            if not words:
+                continue
+            out.append(f"static const uint32_t rf_bp_plan_{th}[] = {{")
+            for i in range(0, len(words), 16):
+                out.append("    " + ", ".join(f"{x}u" for x in words[i:i + 16]) + ",")
+            out.append("};")
+            plans.append(f"{{{th}u, {len(words)}ull, rf_bp_plan_{th}}}")
+    if plans:
+        out.append(f"static const rf_bp_plan_words rf_bp_plans[] = {{{', '.join(plans)}}};")
     out.append("static const rf_design rf_the_design = {")
     out.append(f"    RF_DESIGN_ABI, {comp.opts.block}u, \"{d.name}\", 0x{h:x}ull,")
     out.append(f"    {{{lay.slots['C']}ull, {lay.slots['S']}ull, {lay.slots['I']}ull, {lay.slots['Q']}ull}},")
@@ -1668,7 +1682,8 @@ def emit_descriptor(comp: Compiled, h: int, help_threads: int = 0) -> str:
         out.append("    0, 0ull,")
     mw_w = mw_waves(comp)
     out.append(f"    (const void*)&rf_k_fused_mw, {mw_w}u," if mw_w else "    0, 0u,")
-    out.append(f"    {help_threads}u, (const void*)&rf_k_fused_help" if help_threads else "    0u, 0")
+    out.append(f"    {help_threads}u, (const void*)&rf_k_fused_help," if help_threads else "    0u, 0,")
+    out.append(f"    rf_bp_plans, {len(plans)}u" if plans else "    0, 0u")
     out.append("};")
     # the only exported symbol: kernels stay library-local so several design
     # libraries can live in one process

@@ -73,14 +73,17 @@ struct rf_bp_params {
 };
 
 // Parse and check a blob (every slot index, level table and section size);
-// fills every field but ``a``, ``prog``, ``tab`` and the plan's. Returns 0, or -1
+// fills every field but ``a``, ``prog``, ``tab`` and program M's rounds. Returns 0, or -1
 // with a reason in *why.
 int rf_bp_parse(const uint32_t* blob, uint64_t words, rf_bp_params* p, const char** why);
 
-// Plan program M for ``threads`` threads per workgroup: the plan's words (for
-// p->plan and p->tab) and the fields that describe them. False (nr = 0, the
-// fields left) when it needs more rounds than the kernels hold in registers.
-bool rf_bp_plan(const uint32_t* blob, uint32_t threads, rf_bp_params* p, std::vector<uint32_t>* words);
+// Program M as rounds for ``threads`` threads per workgroup: ``plan`` (a plan
+// in the design's library, ``words`` of it; null: the program's own records)
+// checked against the blob and taken into ``p``, its words for the device in
+// *out (p->tab; p->plan is *rec words further). An empty *out: program M is
+// streamed (nr = 0). Returns 0, or -1 with a reason in *why.
+int rf_bp_plan(const uint32_t* blob, const uint32_t* plan, uint64_t words, uint32_t threads, rf_bp_params* p,
+               std::vector<uint32_t>* out, uint32_t* rec, const char** why);
 
 // The LDS layout behind the planes (tab_off, bal_off) from the table sizes.
 void rf_bp_layout(rf_bp_params* p);

@@ -782,9 +782,6 @@ static bool bp_check_refs(const uint32_t* refs, uint32_t width, uint32_t nslots)
     return true;
 }
 
-// Rounds of register-resident records the kernels of a workgroup size hold.
-static uint32_t bp_max_rounds(uint32_t threads) { return threads < 256 ? 0u : threads >= 1024 ? 40u : RF_BP_MAXR; }
-
 int rf_bp_parse(const uint32_t* b, uint64_t words, rf_bp_params* p, const char** why) {
 #define BP_FAIL(msg)   \
     do {               \
@@ -954,7 +951,8 @@ void rf_bp_layout(rf_bp_params* p) {
     p->bal_off = (bal + 8u <= cu - 64u && cu / planes == cu / (bal + 8u)) ? (uint32_t)bal : 0u;
 }
 
-bool rf_bp_plan(const uint32_t* b, uint32_t threads, rf_bp_params* p, std::vector<uint32_t>* words) {
+int rf_bp_plan(const uint32_t* b, const uint32_t* plan, uint64_t words, uint32_t threads, rf_bp_params* p,
+               std::vector<uint32_t>* out, uint32_t* rec, const char** why) {
     bpplan::Source s{};
     s.blob = b;
     s.byte_form = p->byte_addr != 0;
@@ -973,25 +971,29 @@ bool rf_bp_plan(const uint32_t* b, uint32_t threads, rf_bp_params* p, std::vecto
     s.off_ports = p->off_ports[1];
     p->nr = 0;
     p->bar = 0;
-    const bpplan::Plan pl = bpplan::Planner(s, threads, bp_max_rounds(threads)).run();
-    if (!pl.ok) return false;
-    p->nr = pl.nr;
-    p->bar = pl.bar;
-    words->assign(pl.recs.begin(), pl.recs.end());
-    p->off_cls = (uint32_t)words->size();
-    for (uint64_t c : pl.cls) {
-        words->push_back((uint32_t)c);
-        words->push_back((uint32_t)(c >> 32));
+    out->clear();
+    if (plan) {
+        if (!bpplan::check(s, threads, plan, words)) {
+            *why = "bit-plane plan does not fit its program";
+            return -1;
+        }
+        out->assign(plan, plan + words);
+    } else {
+        const bpplan::Plan own = bpplan::Planner(s, threads, bpplan::max_rounds(threads)).as_stated();
+        if (!own.ok || !own.nr) return 0;
+        *out = bpplan::pack(own, threads);
     }
-    p->off_commit[1] = (uint32_t)words->size();
-    p->n_commit[1] = (uint32_t)pl.commit.size() / 2;
-    words->insert(words->end(), pl.commit.begin(), pl.commit.end());
-    p->off_hash[0] = (uint32_t)words->size();
-    words->insert(words->end(), pl.hash.begin(), pl.hash.end());
-    p->off_ports[1] = (uint32_t)words->size();
-    words->insert(words->end(), pl.ports.begin(), pl.ports.end());
+    const uint32_t* w = out->data();
+    p->nr = w[bpplan::P_NR];
+    p->bar = w[bpplan::P_BAR_LO] | (uint64_t)w[bpplan::P_BAR_HI] << 32;
+    *rec = bpplan::kHdr;
+    p->off_cls = w[bpplan::P_CLS] - bpplan::kHdr;
+    p->off_commit[1] = w[bpplan::P_COMMIT];
+    p->n_commit[1] = w[bpplan::P_NCOMMIT];
+    p->off_hash[0] = w[bpplan::P_HASH];
+    p->off_ports[1] = w[bpplan::P_PORTS];
     rf_bp_layout(p);
-    return true;
+    return 0;
 }
 
 static uint32_t bp_tab_words(const rf_bp_params& p) {

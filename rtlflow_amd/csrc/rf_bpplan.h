@@ -1,6 +1,11 @@
-// rf_bpplan.h -- host planner of the bit-plane kernel's per-cycle program:
-// program M of a blob (generic gate records, level by level) becomes rounds
-// of wavefront rows. Plain C++ (no GPU), so the CPU tests run it.
+// rf_bpplan.h -- planner of the bit-plane kernel's per-cycle program: program
+// M of a blob (generic gate records, level by level) becomes rounds of
+// wavefront rows. Plain C++ (no GPU), so the CPU tests run it. The design's
+// build plans (rf_bpplan.cpp) and writes the plans beside the blob: planning
+// takes about 0.6 us a gate (net2 5 ms), more than a plan saves in 10,000
+// cycles, so no run pays for it. The runtime makes only the unplanned form
+// (as_stated, a copy: 0.02 ms) itself, for workgroup sizes and libraries
+// without a plan.
 //
 // The generic record dst = s ? (x ^ ix) : (y ^ iy) reads three planes and
 // takes 12 VALU instructions whatever the gate is. Here 64 gates of one class
@@ -38,6 +43,7 @@ struct Source {
 
 struct Plan {
     bool ok = false;
+    bool classed = false;              // not just the program's own records
     uint32_t nr = 0;                   // rounds
     uint64_t bar = 0;                  // bit i: a barrier follows round i
     std::vector<uint32_t> recs;        // [round][thread] two words
@@ -47,27 +53,148 @@ struct Plan {
     uint32_t rows = 0, generic = 0;    // wavefront rows, of which generic
 };
 
+// Rounds of register-resident records that the kernels of a workgroup size
+// hold (rf_bitplane.hip).
+inline uint32_t max_rounds(uint32_t threads) { return threads < 256 ? 0u : threads >= 1024 ? 40u : 48u; }
+
+// A plan as words: this header, then at word kHdr the records, the classes,
+// the commit pairs, the hash and the port tables (offsets from the start).
+enum { P_MAGIC, P_THREADS, P_NR, P_BAR_LO, P_BAR_HI, P_CLS, P_COMMIT, P_NCOMMIT, P_HASH, P_PORTS, P_TOTAL };
+constexpr uint32_t kHdr = 12, kMagic = 0x4c504252u;   // 'RBPL'
+inline std::vector<uint32_t> pack(const Plan& p, uint32_t threads) {
+    std::vector<uint32_t> w(kHdr, 0);
+    w[P_MAGIC] = kMagic;
+    w[P_THREADS] = threads;
+    w[P_NR] = p.nr;
+    w[P_BAR_LO] = (uint32_t)p.bar;
+    w[P_BAR_HI] = (uint32_t)(p.bar >> 32);
+    w.insert(w.end(), p.recs.begin(), p.recs.end());
+    w[P_CLS] = (uint32_t)w.size();
+    for (uint64_t c : p.cls) w.insert(w.end(), {(uint32_t)c, (uint32_t)(c >> 32)});
+    w[P_COMMIT] = (uint32_t)w.size();
+    w[P_NCOMMIT] = (uint32_t)p.commit.size() / 2;
+    w.insert(w.end(), p.commit.begin(), p.commit.end());
+    w[P_HASH] = (uint32_t)w.size();
+    w.insert(w.end(), p.hash.begin(), p.hash.end());
+    w[P_PORTS] = (uint32_t)w.size();
+    w.insert(w.end(), p.ports.begin(), p.ports.end());
+    w[P_TOTAL] = (uint32_t)w.size();
+    return w;
+}
+
+// Whether words [w, w + n) are a plan of program M of ``s`` for ``threads``
+// threads: every section inside, every slot a kernel addresses below nslots
+// (a record's fields on rows that run, the tables' references), and tables of
+// the program's own shape.
+inline bool check(const Source& s, uint32_t threads, const uint32_t* w, uint64_t n) {
+    if (n < kHdr || w[P_MAGIC] != kMagic || w[P_THREADS] != threads || w[P_TOTAL] != n || (n >> 31)) return false;
+    const uint32_t nr = w[P_NR], nw = threads / 64;
+    if (!nr || nr > max_rounds(threads) || w[P_CLS] != kHdr + (uint64_t)nr * threads * 2 ||
+        w[P_COMMIT] != w[P_CLS] + (uint64_t)nw * 8 || w[P_HASH] != w[P_COMMIT] + 2ull * w[P_NCOMMIT] ||
+        w[P_PORTS] < w[P_HASH] || w[P_PORTS] > n)
+        return false;
+    if (!((w[nr > 32 ? P_BAR_HI : P_BAR_LO] >> ((nr - 1) % 32)) & 1)) return false;   // the last round ends in a barrier
+    for (uint32_t r = 0; r < nr; ++r)
+        for (uint32_t v = 0; v < nw; ++v) {
+            uint32_t cls = 0;
+            for (uint32_t k = 0; k < 4; ++k) cls |= ((w[w[P_CLS] + 8 * v + 2 * k + r / 32] >> (r % 32)) & 1) << k;
+            if (!(cls & 8)) continue;
+            if ((cls & 7) >= CLASSES) return false;
+            for (uint32_t t = 64 * v; t < 64 * v + 64; ++t) {
+                const uint32_t* g = w + kHdr + 2 * ((uint64_t)r * threads + t);
+                for (uint32_t k = 0; k < 4; ++k) {
+                    uint32_t f = (g[k / 2] >> (16 * (k % 2))) & 0xffffu;
+                    if (s.byte_form ? (k < 2 && (f & 7)) || (f >> 3) >= s.nslots
+                                    : (k < 2 ? f : f & 0x7fffu) >= s.nslots)
+                        return false;
+                }
+            }
+        }
+    const auto slot = [&](uint32_t ref) { return (ref & 0x7fffffffu) < s.nslots; };
+    for (uint32_t k = 0; k < w[P_NCOMMIT]; ++k) {
+        const uint32_t* c = w + w[P_COMMIT] + 2 * k;
+        if (c[0] >= s.nslots || !slot(c[1])) return false;
+    }
+    const uint32_t *b = s.blob + s.off_hash, *h = w + w[P_HASH], *he = w + w[P_PORTS];
+    for (uint32_t k = 0; k < s.n_hash; ++k) {
+        if (he - h < (int64_t)b[1] + 2 || h[0] != b[0] || h[1] != b[1]) return false;
+        for (uint32_t i = 0; i < b[1]; ++i)
+            if (!slot(h[2 + i])) return false;
+        h += 2 + b[1];
+        b += 2 + b[1];
+    }
+    b = s.blob + s.off_ports;
+    const uint32_t* q = w + w[P_PORTS];
+    if (h != he || n - w[P_PORTS] != b[0] || q[0] != b[0] || q[1] != b[1]) return false;
+    uint32_t at = 2;
+    for (uint32_t r = 0; r < b[1]; ++r) {
+        const uint32_t na = b[at + 2], n2 = b[at + 3], refs = b[at] == 0 ? na : 1 + na + n2;
+        const uint32_t size = (b[at] == 0 ? 4u : 5u) + na + n2;
+        for (uint32_t i = 0; i < size; ++i)
+            if (i >= 4 && i < 4 + refs ? !slot(q[at + i]) : q[at + i] != b[at + i]) return false;
+        at += size;
+    }
+    return true;
+}
+
 class Planner {
 public:
-    Planner(const Source& s, uint32_t threads, uint32_t max_rounds)
-        : s_(s), nt_(threads), nw_(threads / 64), maxr_(max_rounds) {}
+    Planner(const Source& s, uint32_t threads, uint32_t rounds)
+        : s_(s), nt_(threads), nw_(threads / 64), maxr_(rounds) {}
 
     // The plan of classed rows; when the program is not of the lowering's form
     // or its values need more slots than it has, its own records as generic
-    // rows. Not ok: more rounds than max_rounds.
+    // rows. Not ok: more rounds than the kernels hold.
     Plan run() {
+        // (a round holds one gate per thread)
+        if (s_.blob[s_.off_lev + s_.nlev] > (uint64_t)nt_ * maxr_) return Plan();
         if (parse() && tables()) {
             for (bool delay : {true, false}) {
                 Plan p;
                 set_levels(delay);
+                if (least_rounds() > maxr_) continue;
                 classify();
                 if (!place(p)) continue;
                 emit_tables(p);
-                p.ok = true;
+                p.ok = p.classed = true;
                 return p;
             }
         }
         return as_stated();
+    }
+
+    // The program's own records as generic rows: no more work than a copy.
+    Plan as_stated() const {
+        Plan p;
+        const uint32_t* b = s_.blob;
+        p.cls.assign((size_t)nw_ * 4, 0);
+        for (uint32_t l = 0; l < s_.nlev; ++l) p.nr += (b[s_.off_lev + l + 1] - b[s_.off_lev + l] + nt_ - 1) / nt_;
+        if (p.nr > maxr_) return Plan();
+        p.recs.resize((size_t)p.nr * nt_ * 2, 0);
+        uint32_t r = 0;
+        for (uint32_t l = 0; l < s_.nlev; ++l) {
+            const uint32_t lo = b[s_.off_lev + l], hi = b[s_.off_lev + l + 1];
+            for (uint32_t k = lo; k < hi; k += nt_, ++r) {
+                const uint32_t n = std::min(hi - k, nt_);
+                uint32_t* rec = &p.recs[(size_t)r * nt_ * 2];
+                std::copy_n(b + s_.off_gates + 2 * k, 2 * n, rec);
+                for (uint32_t w = 0; 64 * w < n; ++w) {
+                    mark(p, w, r, GENERIC);
+                    p.rows++;
+                    p.generic++;
+                }
+                // idle lanes repeat the last record
+                for (uint32_t t = n; t % 64; ++t) std::copy_n(rec + 2 * (n - 1), 2, rec + 2 * t);
+            }
+            if (hi > lo) p.bar |= 1ull << (r - 1);
+        }
+        p.commit.assign(b + s_.off_commit, b + s_.off_commit + 2 * s_.n_commit);
+        uint32_t o = s_.off_hash;
+        for (uint32_t k = 0; k < s_.n_hash; ++k) o += 2 + b[o + 1];
+        p.hash.assign(b + s_.off_hash, b + o);
+        p.ports.assign(b + s_.off_ports, b + s_.off_ports + b[s_.off_ports]);
+        p.ok = true;
+        return p;
     }
 
 private:
@@ -80,7 +207,7 @@ private:
         uint32_t slot = kNone;
         uint32_t target = kNone;      // state slot written in place
         bool keep = false;            // read after the last level
-        std::vector<uint32_t> states; // (state slot << 1 | inverted) that take it
+        uint32_t states = kNone;      // state planes that take it: the first of takes_
         // class row
         uint8_t cls = 0, inv = 0, pol = 0;
         uint32_t s = 0, x = 0, y = 0;
@@ -88,6 +215,15 @@ private:
     struct Field {
         uint32_t dst, s, x, ix, y, iy;
     };
+    struct Take {
+        uint32_t slot, inv, next;   // state slot, inverted; the value's next one in takes_
+    };
+    void add_state(Val& v, uint32_t slot, uint32_t inv) {
+        uint32_t* at = &v.states;   // (kept in the order added: the first that can be is written in place)
+        while (*at != kNone) at = &takes_[*at].next;
+        *at = (uint32_t)takes_.size();
+        takes_.push_back({slot, inv, kNone});
+    }
 
     uint32_t zero() const { return zero_; }
     uint32_t leaf(uint32_t slot) {
@@ -141,6 +277,7 @@ private:
             nfixed_ = std::max(nfixed_, sl[5] + sl[4]);
             for (uint32_t i = 0; i < sl[4]; ++i) is_state_[sl[5] + i] = 1;
         }
+        v_.reserve(b[s_.off_lev + s_.nlev] + nfixed_);
         std::vector<std::pair<uint32_t, uint32_t>> now;
         for (uint32_t l = 0; l < s_.nlev; ++l) {
             now.clear();
@@ -155,7 +292,7 @@ private:
             for (const auto& w : now) {
                 if (w.first < nfixed_) {
                     if (!is_state_[w.first]) return false;
-                    v_[w.second].states.push_back(2 * w.first);
+                    add_state(v_[w.second], w.first, 0);
                 }
                 cur_[w.first] = w.second;
             }
@@ -170,7 +307,7 @@ private:
             const uint32_t* c = b + s_.off_commit + 2 * k;
             const uint32_t v = cur_[c[1] & 0x7fffffffu];
             if (c[0] >= nfixed_ || !is_state_[c[0]] || v == kNone || v_[v].kind == LEAF) return false;
-            v_[v].states.push_back(2 * c[0] + (c[1] >> 31));
+            add_state(v_[v], c[0], c[1] >> 31);
         }
         bool ok = true;
         const auto keep = [&](uint32_t ref) {
@@ -234,9 +371,10 @@ private:
         // their state, so that they can be written in place
         for (int it = 0; it < 2 && delay; ++it) {
             for (Val& v : v_) {
-                if (v.keep || v.states.empty() || v.readers) continue;
+                if (v.keep || v.states == kNone || v.readers) continue;
                 uint32_t want = kNone;
-                for (uint32_t st : v.states) want = std::min(want, last_read(st >> 1) + 1);
+                for (uint32_t k = v.states; k != kNone; k = takes_[k].next)
+                    want = std::min(want, last_read(takes_[k].slot) + 1);
                 v.level = std::min(lmax_, std::max(v.asap, want));
             }
             scan();
@@ -246,12 +384,23 @@ private:
             scan();
         }
         for (Val& v : v_) {
-            for (uint32_t st : v.states)
-                if (v.target == kNone && !(st & 1) && last_read(st >> 1) < v.level) v.target = st >> 1;
+            for (uint32_t k = v.states; k != kNone; k = takes_[k].next)
+                if (v.target == kNone && !takes_[k].inv && last_read(takes_[k].slot) < v.level) v.target = takes_[k].slot;
             if (v.keep) v.last = lmax_ + 1;
-            for (uint32_t st : v.states)
-                if ((st >> 1) != v.target) v.last = lmax_ + 1;
+            for (uint32_t k = v.states; k != kNone; k = takes_[k].next)
+                if (takes_[k].slot != v.target) v.last = lmax_ + 1;
         }
+    }
+
+    // Rounds that the levels need at the least (classes that leave wavefront
+    // rows partly empty can need more).
+    uint32_t least_rounds() const {
+        std::vector<uint32_t> n(lmax_ + 1, 0);
+        for (const Val& v : v_)
+            if (v.kind != LEAF) n[v.level]++;
+        uint32_t r = 0;
+        for (uint32_t x : n) r += (x + nt_ - 1) / nt_;
+        return r;
     }
 
     // A level's rows past its last full round of threads move on to the next
@@ -336,6 +485,7 @@ private:
         std::vector<std::vector<uint32_t>> free(32);
         uint32_t top = nfixed_;
         count_banks();
+        banks_.assign(4, Banks(s_.nslots));
         p.cls.assign((size_t)nw_ * 4, 0);
         for (uint32_t l = 1; l <= lmax_; ++l) {
             // temporaries last read at an earlier level are free
@@ -344,11 +494,11 @@ private:
             for (uint32_t i : at[l]) grp[v_[i].inv ? (uint32_t)GENERIC : v_[i].cls].push_back(i);
             pool_remainders(grp);
             std::vector<std::pair<uint32_t, std::vector<uint32_t>>> wr;   // class, values
-            for (uint32_t c = 0; c < CLASSES; ++c)
-                for (size_t k = 0; k < grp[c].size(); k += 64) {
-                    spread(grp[c], k, c);
+            for (uint32_t c = 0; c < CLASSES; ++c) {
+                spread(grp[c], c);
+                for (size_t k = 0; k < grp[c].size(); k += 64)
                     wr.push_back({c, {grp[c].begin() + k, grp[c].begin() + std::min(grp[c].size(), k + 64)}});
-                }
+            }
             const uint32_t rounds = ((uint32_t)wr.size() + nw_ - 1) / nw_;
             if (p.nr + rounds > maxr_) return false;
             p.recs.resize((size_t)(p.nr + rounds) * nt_ * 2, 0);
@@ -394,39 +544,6 @@ private:
     static void mark(Plan& p, uint32_t wave, uint32_t round, uint32_t cls) {
         for (uint32_t bit = 0; bit < 4; ++bit)
             if (((cls | 8u) >> bit) & 1) p.cls[4 * wave + bit] |= 1ull << round;
-    }
-
-    // The program's own records as generic rows.
-    Plan as_stated() const {
-        Plan p;
-        const uint32_t* b = s_.blob;
-        p.cls.assign((size_t)nw_ * 4, 0);
-        for (uint32_t l = 0; l < s_.nlev; ++l) {
-            const uint32_t lo = b[s_.off_lev + l], hi = b[s_.off_lev + l + 1];
-            for (uint32_t k = lo; k < hi; k += nt_, ++p.nr) {
-                if (p.nr >= maxr_) return Plan();
-                p.recs.resize((size_t)(p.nr + 1) * nt_ * 2, 0);
-                for (uint32_t w = 0; w < nw_ && k + 64 * w < hi; ++w) {
-                    mark(p, w, p.nr, GENERIC);
-                    p.rows++;
-                    p.generic++;
-                    for (uint32_t t = 0; t < 64; ++t) {
-                        const uint32_t* g = b + s_.off_gates + 2 * std::min(k + 64 * w + t, hi - 1);
-                        uint32_t* rec = &p.recs[((size_t)p.nr * nt_ + w * 64 + t) * 2];
-                        rec[0] = g[0];
-                        rec[1] = g[1];
-                    }
-                }
-            }
-            if (hi > lo) p.bar |= 1ull << (p.nr - 1);
-        }
-        p.commit.assign(b + s_.off_commit, b + s_.off_commit + 2 * s_.n_commit);
-        uint32_t o = s_.off_hash;
-        for (uint32_t k = 0; k < s_.n_hash; ++k) o += 2 + b[o + 1];
-        p.hash.assign(b + s_.off_hash, b + o);
-        p.ports.assign(b + s_.off_ports, b + s_.off_ports + b[s_.off_ports]);
-        p.ok = true;
-        return p;
     }
 
     // Classes' last rows that do not fill a wavefront row become generic,
@@ -487,34 +604,45 @@ private:
     }
     void count_banks() {
         use_.assign((size_t)(lmax_ + 1) * CLASSES * 3 * 32, 0);
-        readers_.assign(v_.size(), {});
-        for (uint32_t i = 0; i < v_.size(); ++i) {
-            Val& v = v_[i];
-            if (v.kind == LEAF) continue;
-            const uint32_t op[3] = {v.s, v.x, v.y};
-            for (uint32_t k = 0; k < reads(v); ++k) {
-                const Val& x = v_[op[k]];
-                if (x.kind == LEAF || x.target != kNone)
-                    bank_use(v, k)[(x.kind == LEAF ? x.slot : x.target) % 32]++;
-                else
-                    readers_[op[k]].push_back(4 * i + k);
+        rd_at_.assign(v_.size() + 1, 0);
+        const auto each = [&](const auto& fn) {
+            for (Val& v : v_) {
+                if (v.kind == LEAF) continue;
+                const uint32_t op[3] = {v.s, v.x, v.y};
+                for (uint32_t k = 0; k < reads(v); ++k) fn(v, k, op[k]);
             }
-        }
+        };
+        each([&](Val& v, uint32_t k, uint32_t i) {
+            const Val& x = v_[i];
+            if (x.kind == LEAF || x.target != kNone)
+                bank_use(v, k)[(x.kind == LEAF ? x.slot : x.target) % 32]++;
+            else
+                ++rd_at_[i + 1];
+        });
+        for (size_t i = 1; i < rd_at_.size(); ++i) rd_at_[i] += rd_at_[i - 1];
+        rd_use_.resize(rd_at_.back());
+        std::vector<uint32_t> to(rd_at_);
+        each([&](Val& v, uint32_t k, uint32_t i) {
+            if (v_[i].kind != LEAF && v_[i].target == kNone) rd_use_[to[i]++] = (uint32_t)(bank_use(v, k) - use_.data());
+        });
     }
     // A slot for value ``i``: a free one or the next new one, its bank pair
     // not in ``held`` (the destinations of its 32 lanes).
     uint32_t take(std::vector<std::vector<uint32_t>>& free, uint32_t held, uint32_t& top, uint32_t i) {
+        uint32_t cost[32];
+        for (uint32_t r = 0; r < 32; ++r) cost[r] = 63 - (uint32_t)std::min<size_t>(63, free[r].size());
+        for (uint32_t k = rd_at_[i]; k < rd_at_[i + 1]; ++k) {
+            const uint32_t* u = &use_[rd_use_[k]];
+            for (uint32_t r = 0; r < 32; ++r) cost[r] += 64 * u[r];
+        }
         uint32_t best = kNone, least = kNone;
         for (int any = held == kNone ? 1 : 0; any < 2 && best == kNone; ++any)
             for (uint32_t r = 0; r < 32; ++r) {
                 if ((((held >> r) & 1) && !any) || (free[r].empty() && top + 32 > s_.nslots)) continue;
-                uint32_t c = 0;
-                for (uint32_t rd : readers_[i]) c += bank_use(v_[rd / 4], rd % 4)[r];
-                c = c * 64 + 63 - (uint32_t)std::min<size_t>(63, free[r].size());
-                if (c < least) least = c, best = r;
+                if (cost[r] < least) least = cost[r], best = r;
             }
         if (best == kNone) return top++;   // past the program's slots: the plan fails
-        for (uint32_t rd : readers_[i]) bank_use(v_[rd / 4], rd % 4)[best]++;
+        for (uint32_t k = rd_at_[i]; k < rd_at_[i + 1]; ++k) use_[rd_use_[k] + best]++;
         if (free[best].empty()) {
             while (top % 32 != best) {
                 free[top % 32].push_back(top);
@@ -531,66 +659,74 @@ private:
     // 64-bit accesses at a time, in as many passes as the most slots that
     // differ in one bank pair (slot modulo 32; equal slots are one access).
     struct Banks {
-        uint32_t slot[32][8];
+        std::vector<uint32_t> at;   // per slot: the set it was last put in
+        uint32_t set = 0;
         uint8_t n[32];
         uint8_t most;
+        explicit Banks(uint32_t nslots) : at(nslots, 0) {}
         void clear() {
+            ++set;
             std::fill(n, n + 32, 0);
             most = 0;
         }
-        bool has(uint32_t s) const {
-            const uint32_t r = s % 32;
-            for (uint32_t i = 0; i < n[r]; ++i)
-                if (slot[r][i] == s) return true;
-            return false;
-        }
         // 256 for another pass, plus the slots already in the bank pair
         uint32_t cost(uint32_t s) const {
-            if (has(s)) return 0;
+            if (at[s] == set) return 0;
             const uint32_t c = n[s % 32];
             return c + (c == most ? 256u : 0u);
         }
         void put(uint32_t s) {
-            const uint32_t r = s % 32;
-            if (has(s)) return;
-            if (n[r] < 8) slot[r][n[r]++] = s;
-            most = std::max(most, n[r]);
+            if (at[s] == set) return;
+            at[s] = set;
+            most = std::max(most, ++n[s % 32]);
         }
     };
 
-    // Rows g[k0 .. k0 + 64) chosen from g[k0 ..) and ordered: each next row is
-    // the one whose operands (and fixed destination) need the fewest further
-    // passes of the current 32 lanes; a commutative gate's operands may swap.
-    void spread(std::vector<uint32_t>& g, size_t k0, uint32_t cls) {
-        Banks bk[4];
-        const size_t end = std::min(g.size(), k0 + 64);
-        for (size_t k = k0; k < end; ++k) {
-            if ((k - k0) % 32 == 0)
-                for (Banks& b : bk) b.clear();
+    // The rows of a class of a level ordered: each next row is the one whose
+    // operands (and fixed destination) need the fewest further passes of the
+    // current 32 lanes; a commutative gate's operands may swap.
+    void spread(std::vector<uint32_t>& g, uint32_t cls) {
+        struct Cand {
+            uint32_t s, x, y, dst, val;
+        };
+        std::vector<Cand> left(g.size());
+        for (size_t k = 0; k < g.size(); ++k) {
+            const Val& v = v_[g[k]];
+            const Field f = cls == GENERIC ? generic(v) : plain(v);
+            left[k] = {f.s, f.x, f.y, v.target, g[k]};
+        }
+        const bool swaps = cls == AND || cls == NOR || cls == XOR, three = cls >= MUX;
+        Banks &bs = banks_[0], &bx = banks_[1], &by = banks_[2], &bd = banks_[3];
+        for (size_t k = 0; k < left.size(); ++k) {
+            if (k % 32 == 0)
+                for (Banks& b : banks_) b.clear();
             size_t best = k;
             uint32_t least = kNone;
             bool swap = false;
-            for (size_t j = k; j < g.size() && least; ++j) {
-                const Val& v = v_[g[j]];
-                const Field f = cls == GENERIC ? generic(v) : plain(v);
-                uint32_t c = v.target != kNone ? bk[3].cost(v.target) : 0u;
-                if (cls >= MUX) c += bk[2].cost(f.y);
-                const uint32_t c0 = c + bk[0].cost(f.s) + bk[1].cost(f.x);
-                if (c0 < least) least = c0, best = j, swap = false;
-                if (cls == AND || cls == NOR || cls == XOR) {
-                    const uint32_t c1 = c + bk[0].cost(f.x) + bk[1].cost(f.s);
-                    if (c1 < least) least = c1, best = j, swap = true;
+            // (the first row of a half: any)
+            const size_t end = k % 32 ? left.size() : k + 1;
+            for (size_t j = k; j < end && least; ++j) {
+                const Cand& c = left[j];
+                uint32_t w = c.dst != kNone ? bd.cost(c.dst) : 0u;
+                if (three) w += by.cost(c.y);
+                const uint32_t w0 = w + bs.cost(c.s) + bx.cost(c.x);
+                if (w0 < least) least = w0, best = j, swap = false;
+                if (swaps) {
+                    const uint32_t w1 = w + bs.cost(c.x) + bx.cost(c.s);
+                    if (w1 < least) least = w1, best = j, swap = true;
                 }
-                if ((k - k0) % 32 == 0) break;   // the first row of a half: any
             }
-            std::swap(g[k], g[best]);
-            Val& v = v_[g[k]];
-            if (swap) std::swap(v.s, v.x);
-            const Field f = cls == GENERIC ? generic(v) : plain(v);
-            if (v.target != kNone) bk[3].put(v.target);
-            if (cls >= MUX) bk[2].put(f.y);
-            bk[0].put(f.s);
-            bk[1].put(f.x);
+            std::swap(left[k], left[best]);
+            Cand& c = left[k];
+            if (swap) {
+                std::swap(c.s, c.x);
+                std::swap(v_[c.val].s, v_[c.val].x);
+            }
+            if (c.dst != kNone) bd.put(c.dst);
+            if (three) by.put(c.y);
+            bs.put(c.s);
+            bx.put(c.x);
+            g[k] = c.val;
         }
     }
 
@@ -603,8 +739,8 @@ private:
         const uint32_t* b = s_.blob;
         std::vector<std::pair<uint32_t, uint32_t>> com;
         for (const Val& v : v_)
-            for (uint32_t st : v.states)
-                if ((st >> 1) != v.target) com.push_back({st >> 1, v.slot | ((st & 1) ^ v.pol) << 31});
+            for (uint32_t k = v.states; k != kNone; k = takes_[k].next)
+                if (takes_[k].slot != v.target) com.push_back({takes_[k].slot, v.slot | (takes_[k].inv ^ v.pol) << 31});
         spread_commit(com);
         for (const auto& c : com) p.commit.insert(p.commit.end(), {c.first, c.second});
         uint32_t o = s_.off_hash;
@@ -624,8 +760,8 @@ private:
     }
     // Commit pairs ordered like rows: reads and writes of each 32 spread over
     // the bank pairs.
-    static void spread_commit(std::vector<std::pair<uint32_t, uint32_t>>& c) {
-        Banks bk[2];
+    void spread_commit(std::vector<std::pair<uint32_t, uint32_t>>& c) const {
+        std::vector<Banks> bk(2, Banks(s_.nslots));
         for (size_t k = 0; k < c.size(); ++k) {
             if (k % 32 == 0) bk[0].clear(), bk[1].clear();
             size_t best = k;
@@ -643,10 +779,12 @@ private:
     const Source s_;
     const uint32_t nt_, nw_, maxr_;
     std::vector<Val> v_;
+    std::vector<Take> takes_;
     std::vector<uint32_t> cur_;     // slot -> value it holds
     std::vector<char> is_state_;
     std::vector<uint32_t> use_;                    // bank_use()
-    std::vector<std::vector<uint32_t>> readers_;   // of a temporary: 4 * value + operand
+    std::vector<uint32_t> rd_at_, rd_use_;         // of a temporary i: its readers' rows of use_, rd_use_[rd_at_[i] ..)
+    std::vector<Banks> banks_;                     // of spread(): s, x, y, fixed destinations
     uint32_t nfixed_ = 0, lmax_ = 0, zero_ = kNone;
 };
 

@@ -98,8 +98,7 @@ struct rf_model {
     rf_stats stats{};
     rf_args base{};
     uint32_t* bp_prog = nullptr;   // device copy of the bit-plane program
-    uint32_t* bp_plan = nullptr;   // the plan of its per-cycle program, made on first use
-    bool bp_planned = false;
+    uint32_t* bp_tab = nullptr;    // and of its per-cycle program's rounds
     unsigned long long* bp_progress = nullptr;  // progress counter of a bit-plane launch
     int bp_per_cu[2] = {0, 0};     // bit-plane workgroups per CU (plain / stream kernel), 0 = not asked yet
     rf_bp_params bp{};
@@ -291,25 +290,26 @@ int load_bitplane(rf_model* m) {
         if (me[2] ? loc + md.row_bytes > d->mem_row_bytes : loc + md.depth > d->slots[md.cls])
             return fail(RF_E_DESIGN, "bit-plane memory %s outside the layout", md.name);
     }
-    const size_t bytes = d->bitplane_words * 4;
-    RF_HIP(hipMalloc(&m->bp_prog, bytes));
-    RF_HIP(hipMemcpy(m->bp_prog, b, bytes, hipMemcpyHostToDevice));
+    // the library's plan of the per-cycle program for this workgroup size
+    const uint32_t th = m->cfg.bitplane_threads;
+    const uint32_t* plan = nullptr;
+    uint64_t pwords = 0;
+    for (uint32_t k = 0; d->abi >= 10u && k < d->n_bp_plans; ++k)
+        if (d->bp_plans[k].threads == th) plan = d->bp_plans[k].words, pwords = d->bp_plans[k].n;
+    std::vector<uint32_t> tab;
+    uint32_t rec = 0;
+    if (rf_bp_plan(b, plan, pwords, th, &m->bp, &tab, &rec, &why)) return fail(RF_E_DESIGN, "%s", why);
+    RF_HIP(hipMalloc(&m->bp_prog, d->bitplane_words * 4));
+    RF_HIP(hipMemcpy(m->bp_prog, b, d->bitplane_words * 4, hipMemcpyHostToDevice));
     m->bp.prog = m->bp.tab = m->bp_prog;
+    if (!tab.empty()) {
+        RF_HIP(hipMalloc(&m->bp_tab, tab.size() * 4));
+        RF_HIP(hipMemcpy(m->bp_tab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
+        m->bp.tab = m->bp_tab;
+        m->bp.plan = m->bp_tab + rec;
+    }
     RF_HIP(hipMalloc(&m->bp_progress, sizeof(unsigned long long)));
     m->bp.progress = m->bp_progress;
-    return RF_OK;
-}
-
-// Plan the per-cycle program on the model's first bit-plane run.
-int plan_bitplane(rf_model* m) {
-    if (m->bp_planned) return RF_OK;
-    std::vector<uint32_t> words;
-    if (rf_bp_plan(m->d->bitplane, m->cfg.bitplane_threads, &m->bp, &words)) {
-        RF_HIP(hipMalloc(&m->bp_plan, words.size() * 4));
-        RF_HIP(hipMemcpy(m->bp_plan, words.data(), words.size() * 4, hipMemcpyHostToDevice));
-        m->bp.plan = m->bp.tab = m->bp_plan;
-    }
-    m->bp_planned = true;
     return RF_OK;
 }
 
@@ -540,7 +540,7 @@ uint64_t rf_lane_stride(const rf_model* m) { return m ? m->npad : 0; }
 int rf_create(const rf_design* d, uint32_t n_lanes, const rf_config* cfg, rf_model** out) {
     if (!d || !out) return fail(RF_E_ARG, "rf_create: null design or output pointer");
     *out = nullptr;
-    if (d->abi != RF_DESIGN_ABI && d->abi != 8u)   // 8: no k_fused_help
+    if (d->abi != RF_DESIGN_ABI && d->abi != 8u && d->abi != 9u)   // 8: no k_fused_help; 9: no bit-plane plans
         return fail(RF_E_DESIGN, "design ABI %u, runtime expects %u", d->abi, RF_DESIGN_ABI);
     if (n_lanes == 0) return fail(RF_E_ARG, "rf_create: n_lanes must be > 0");
     if (cfg && cfg->bitplane_threads &&
@@ -668,7 +668,7 @@ int rf_destroy(rf_model* m) {
     for (int c = 0; c < 4; ++c)
         if (m->cls[c]) (void)hipFree(m->cls[c]);
     void* ps[] = {m->mem, m->change, m->done, m->hash, m->cyc, m->stim, m->flags,
-                  m->budget, m->order, m->out_hash, m->images, m->bp_prog, m->bp_plan, m->bp_progress};
+                  m->budget, m->order, m->out_hash, m->images, m->bp_prog, m->bp_tab, m->bp_progress};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     for (void* p : m->image_bufs)
@@ -918,10 +918,6 @@ int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
     if (rc) return rc;
     rc = do_init(m);
     if (rc) return rc;
-    if (mode == RF_MODE_BITPLANE) {
-        rc = plan_bitplane(m);
-        if (rc) return rc;
-    }
     hipEvent_t e0;
     if (mode == RF_MODE_GRAPH) {
         if (!n) return RF_OK;
@@ -1378,8 +1374,7 @@ int rf_submit_queue_static(rf_model* m, uint64_t seed, const uint32_t* budgets, 
 // whole queue's size, for the kernel's budget lookups).
 static int bitplane_rounds(rf_model* m, uint64_t seed, const uint32_t* budgets, const uint32_t* ord,
                            uint32_t n, uint32_t nstim) {
-    int rc = plan_bitplane(m);
-    if (rc) return rc;
+    int rc = RF_OK;
     const uint32_t nl = m->nlanes;
     std::vector<uint64_t> h(m->npad, 0xcbf29ce484222325ull);
     std::vector<uint32_t> sid(m->npad, 0);

@@ -11,7 +11,8 @@ import numpy as np
 import pytest
 
 from rtlflow_amd import bitplane as bp
-from rtlflow_amd.compiler import Compiled, Options
+from rtlflow_amd.build import build_planner
+from rtlflow_amd.compiler import Compiled, Options, emit_source
 from rtlflow_amd.designs import rams
 from rtlflow_amd.designs.fuzz import verilog as fuzz
 from rtlflow_amd.designs.netlist import generate
@@ -82,3 +83,69 @@ def test_programs_of_another_form_keep_their_records(host):
     blob[sec["hashM"] + 2] = blob[sec["commitM"]]
     rc, (a, b), info = plan_run(host, blob, 256, np.random.default_rng(1))
     assert rc == 0 and (a == b).all() and info[1] == info[2]
+
+
+def _design(name="b"):
+    src = generate(n_gates=400, n_ff=40, n_pi=16, n_po=24, depth=10, seed=7, n_rams=1, ram_depth=8, ram_width=4,
+                   name=name)[0]
+    return Compiled(elaborate(src), Options(threads=2))
+
+
+def test_design_libraries_carry_their_plans():
+    """Planning belongs to the design's build: the emitted source holds the
+    plan of every workgroup size that has one, so no model and no run makes
+    it."""
+    comp = _design()
+    text = emit_source(comp)
+    for th in bp.PLAN_THREADS:
+        words = bp.plan(comp.bitplane_blob, th)
+        assert words and f"static const uint32_t rf_bp_plan_{th}[] = {{\n    {words[0]}u, {th}u, {words[2]}u," in text
+        assert f"{{{th}u, {len(words)}ull, rf_bp_plan_{th}}}" in text
+    assert f"    rf_bp_plans, {len(bp.PLAN_THREADS)}u\n" in text
+
+
+@pytest.mark.parametrize("byte_form", [True, False])
+def test_plans_are_checked_against_their_program(byte_form, monkeypatch):
+    """A plan's words pass the check that the runtime makes; a slot, a class,
+    a table or a size out of range does not."""
+    if not byte_form:
+        monkeypatch.setattr(bp, "BYTE_FORM_MAX_SLOTS", 0)
+    blob = _design().bitplane_blob
+    lib = C.CDLL(str(build_planner()))
+    b = np.asarray(blob, np.uint32)
+    sec = bp.sections(blob)
+    s = np.array([sec[k] for k in bp._PLAN_SECTIONS], np.uint32)
+    ptr = lambda a: a.ctypes.data_as(C.c_void_p)
+    check = lambda w, th=256: lib.rf_bpplan_check(ptr(b), ptr(s), th, ptr(w), C.c_uint64(len(w)))
+    w = np.array(bp.plan(blob, 256), np.uint32)
+    assert check(w)
+    assert not check(w, 512) and not check(w[:-1]) and not check(w[:8])
+    nr, cls, commit, ncom, hsh, ports = (int(w[k]) for k in (2, 5, 6, 7, 8, 9))
+    big = int(b[2]) * (8 if byte_form else 1)      # the first slot past the planes
+
+    def bad(at, value):
+        v = w.copy()
+        v[at] = value
+        return not check(v)
+
+    def row(wave, r):                              # first record of the first wavefront row that runs
+        return 12 + 2 * (r * 256 + 64 * wave)
+
+    runs = [(wv, r) for wv in range(4) for r in range(nr)
+            if (int(w[cls + 8 * wv + 6 + r // 32]) >> (r % 32)) & 1]
+    at = row(*runs[0])
+    assert bad(at, (int(w[at]) & 0xffff0000) | big) and bad(at, (int(w[at]) & 0xffff) | big << 16)
+    if big < 0x8000:
+        assert bad(at + 1, (int(w[at + 1]) & 0xffff0000) | big) and bad(at + 1, big << 16)
+    assert bad(2, nr + 1) and bad(2, 0) and bad(2, 49)
+    assert bad(3, int(w[3]) & ~(1 << (nr - 1)))
+    wv, r = runs[0]
+    w2 = w.copy()
+    for q in range(3):                             # class 7
+        w2[cls + 8 * wv + 2 * q] |= 1 << r
+    assert not check(w2)
+    assert ncom and bad(commit, int(b[2])) and bad(commit + 1, int(b[2])) and bad(commit + 1, 0x80000000 | int(b[2]))
+    assert bad(hsh, int(w[hsh]) ^ 1) and bad(hsh + 2, int(b[2])) and bad(ports + 1, int(w[ports + 1]) + 1)
+    assert bad(ports + 6, int(b[2])) and bad(ports + 3, 99)
+    for k in (5, 6, 7, 8, 9, 10):
+        assert bad(k, int(w[k]) + 1) and bad(k, 0xffffffff)
