@@ -11,7 +11,9 @@ GPU is present, constructing a model raises.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import json
+import sys
 from pathlib import Path
 from typing import Dict, List, Optional, Sequence, Tuple, Union
 
@@ -53,6 +55,23 @@ class rf_stream(C.Structure):
 _rt = None
 
 
+def _one_hip_runtime():
+    """Load the HIP runtime that torch ships, if torch is installed, before
+    the runtime library asks for one: torch brings its own copy, and a process
+    that loads the system's first holds two from its ``import torch`` on. The
+    model's runtime would then not know torch's tensors (stream and capture
+    buffers), and two runtimes would share one GPU's queues and one process's
+    exit. With the copy already loaded both take it, in either order."""
+    if "torch" in sys.modules:
+        return
+    spec = importlib.util.find_spec("torch")
+    for d in (spec.submodule_search_locations if spec else None) or []:
+        hip = Path(d) / "lib" / "libamdhip64.so"
+        if hip.exists():
+            C.CDLL(str(hip))
+            return
+
+
 def runtime() -> C.CDLL:
     """Load librf_verilated.so and declare its entry points."""
     global _rt
@@ -61,6 +80,7 @@ def runtime() -> C.CDLL:
     path = runtime_path()
     if not path.exists():
         raise RFError(f"runtime library {path} is not built; run __graft_entry__.build()")
+    _one_hip_runtime()
     lib = C.CDLL(str(path), mode=C.RTLD_GLOBAL)
     P = C.c_void_p
     u32, u64 = C.c_uint32, C.c_uint64
