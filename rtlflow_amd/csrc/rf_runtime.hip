@@ -100,6 +100,7 @@ struct rf_model {
     uint32_t* bp_prog = nullptr;   // device copy of the bit-plane program
     uint32_t* bp_tab = nullptr;    // and of its per-cycle program's rounds
     unsigned long long* bp_progress = nullptr;  // progress counter of a bit-plane launch
+    uint32_t help_groups = 0;      // groups of 64 stimuli that k_fused_help takes, 0 = not asked yet
     int bp_per_cu[2] = {0, 0};     // bit-plane workgroups per CU (plain / stream kernel), 0 = not asked yet
     rf_bp_params bp{};
     // launches of rf_run_cycles not yet waited for: their HIP events are
@@ -901,12 +902,23 @@ static std::vector<bp_window> bp_rotation(uint32_t G, uint32_t S, uint32_t n, bo
 }
 
 // The fused form with helper wavefronts: up to four groups of 64 stimuli per CU,
-// which its LDS holds at once (the register-file ALU, 4,000 cycles, 256 CUs: four
-// groups a CU 3.0 ms -> 1.68, one 2.9 -> 0.81). Above that the groups would run
-// in rounds; the plain kernel's one wavefront per group fills the SIMDs.
-static bool helped(const rf_model* m) {
-    return m->d->abi >= 9u && m->d->k_fused_help && !streams_set(m) &&
-           (m->nlanes + 63u) / 64u <= 4u * (uint32_t)std::max(1, m->ncu);
+// or as many as its LDS holds at once. Above that the groups would run in
+// rounds; the plain kernel's one wavefront per group fills the SIMDs. Measured,
+// 2,000 cycles, one group a CU and four, plain -> helped: the register-file ALU
+// 1.33 -> 0.38 and 1.32 -> 0.79 ms; a gated-clock counter 0.44 -> 0.19 and 0.52 ->
+// 0.37; small word-level designs 0.95 -> 0.56 and 1.00 -> 0.67 (reductions), 0.96 ->
+// 0.51 and 0.97 -> 0.61 (signed), 5.42 -> 5.24 and 5.43 -> 5.35 (wide shifts, whose
+// own logic is nearly all of a cycle).
+static int helped(rf_model* m, bool* yes) {
+    *yes = false;
+    if (m->d->abi < 9u || !m->d->k_fused_help || streams_set(m)) return RF_OK;
+    if (!m->help_groups) {
+        int n = 0;
+        RF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, m->d->k_fused_help, (int)m->d->help_threads, 0));
+        m->help_groups = (uint32_t)std::max(1, std::min(4, n)) * (uint32_t)std::max(1, m->ncu);
+    }
+    *yes = (m->nlanes + 63u) / 64u <= m->help_groups;
+    return RF_OK;
 }
 
 int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
@@ -936,13 +948,16 @@ int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
         if (mode == RF_MODE_FUSED) {
             rf_args a = args_for(m, RF_PHASE_EVAL);
             a.ncycles = chunk;
+            bool help;
+            rc = helped(m, &help);
+            if (rc) return rc;
             if (m->cfg.fused_multiwave && m->d->k_fused_mw && m->d->mw_waves >= 2 && m->d->mw_waves <= 16 &&
                 !streams_set(m)) {
                 // one workgroup of mw_waves wavefronts per 64 stimuli
                 void* params[] = {&a};
                 RF_HIP(hipLaunchKernel(m->d->k_fused_mw, dim3((m->nlanes + 63u) / 64u), dim3(64u * m->d->mw_waves),
                                        params, 0, m->stream));
-            } else if (helped(m)) {
+            } else if (help) {
                 void* params[] = {&a};
                 RF_HIP(hipLaunchKernel(m->d->k_fused_help, dim3((m->nlanes + 63u) / 64u), dim3(m->d->help_threads),
                                        params, 0, m->stream));
