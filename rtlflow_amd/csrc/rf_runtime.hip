@@ -218,17 +218,22 @@ int add_eval(rf_model* m, hipGraph_t g, hipGraphNode_t dep, uint32_t unroll, uin
     return RF_OK;
 }
 
-int build_graphs(rf_model* m) {
-    const rf_design* d = m->d;
+// One eval, a settle iteration per replay (rf_eval).
+int build_eval_graph(rf_model* m) {
     // argument blocks must outlive node creation only (kernel params are copied)
     std::deque<rf_args> argstore;
-    // eval graph: one eval (used by rf_eval, one settle iteration per replay)
     RF_HIP(hipGraphCreate(&m->eval_graph, 0));
     hipGraphNode_t tail;
     int rc = add_eval(m, m->eval_graph, nullptr, 1, RF_PHASE_EVAL, false, argstore, &tail);
     if (rc) return rc;
     RF_HIP(hipGraphInstantiate(&m->eval_exec, m->eval_graph, nullptr, nullptr, 0));
-    // cycle graph: stim -> eval(clk=0) -> rise -> eval(clk=1) -> hash
+    return RF_OK;
+}
+
+// One clock cycle: stim -> eval(clk=0) -> rise -> eval(clk=1) -> hash.
+int build_cycle_graph(rf_model* m) {
+    const rf_design* d = m->d;
+    std::deque<rf_args> argstore;
     RF_HIP(hipGraphCreate(&m->cycle_graph, 0));
     hipKernelNodeParams p{};
     p.func = const_cast<void*>(d->k_stim);
@@ -242,7 +247,7 @@ int build_graphs(rf_model* m) {
     const uint32_t unroll = d->nchange ? std::max<uint32_t>(1, m->cfg.settle_unroll) : 1;
     const bool settle_tail = d->nchange && d->k_settle;
     hipGraphNode_t t1, t2;
-    rc = add_eval(m, m->cycle_graph, stim, unroll, RF_PHASE_RISE, settle_tail, argstore, &t1);
+    int rc = add_eval(m, m->cycle_graph, stim, unroll, RF_PHASE_RISE, settle_tail, argstore, &t1);
     if (rc) return rc;
     rc = add_eval(m, m->cycle_graph, t1, unroll, RF_PHASE_HASH, settle_tail, argstore, &t2);
     if (rc) return rc;
@@ -408,14 +413,19 @@ void drop_graphs(rf_model* m) {
     m->eval_graph = nullptr;
 }
 
-// Rebuild the graphs when their kernel arguments are out of date.
-int fresh_graphs(rf_model* m) {
-    if (!m->graphs_stale && m->cycle_exec) return RF_OK;
-    drop_graphs(m);
-    int rc = build_graphs(m);
-    if (rc) return rc;
+// The graph of one clock cycle (``cycle``) or of one eval, built where a call
+// first needs it and again when its kernel arguments are out of date: a model
+// that runs in another form instantiates none.
+int fresh_graph(rf_model* m, bool cycle) {
+    if (m->graphs_stale && (m->cycle_exec || m->eval_exec)) {
+        RF_HIP(hipStreamSynchronize(m->stream));   // no replay of theirs may be in flight
+        drop_graphs(m);
+    }
     m->graphs_stale = false;
-    return RF_OK;
+    if (cycle ? m->cycle_exec : m->eval_exec) return RF_OK;
+    const int rc = cycle ? build_cycle_graph(m) : build_eval_graph(m);
+    if (rc) drop_graphs(m);
+    return rc;
 }
 
 // Wait for every queued launch, fold the HIP-event times into the
@@ -647,10 +657,8 @@ int rf_create(const rf_design* d, uint32_t n_lanes, const rf_config* cfg, rf_mod
     e = hipEventCreate(&m->ev0);
     if (e == hipSuccess) e = hipEventCreate(&m->ev1);
     if (e != hipSuccess) return cleanup(fail(RF_E_HIP, "hipEventCreate: %s", hipGetErrorString(e)));
-    int rc = build_graphs(m);
-    if (rc) return cleanup(rc);
     if (d->bitplane && d->bitplane_words) {
-        rc = load_bitplane(m);
+        const int rc = load_bitplane(m);
         if (rc) return cleanup(rc);
     }
     *out = m;
@@ -804,7 +812,7 @@ int rf_eval(rf_model* m) {
     }
     int rc = do_init(m);
     if (rc) return rc;
-    rc = fresh_graphs(m);
+    rc = fresh_graph(m, false);
     if (rc) return rc;
     const rf_design* d = m->d;
     if (!d->nchange) {
@@ -933,7 +941,7 @@ int rf_run_cycles(rf_model* m, uint32_t n, uint32_t mode) {
     hipEvent_t e0;
     if (mode == RF_MODE_GRAPH) {
         if (!n) return RF_OK;
-        rc = fresh_graphs(m);
+        rc = fresh_graph(m, true);
         if (rc) return rc;
         rc = timed_begin(m, &e0);
         if (rc) return rc;

@@ -1,3 +1,5 @@
+import ctypes
+import subprocess
 import sys
 from pathlib import Path
 
@@ -14,9 +16,14 @@ def pytest_configure(config):
 
 
 @pytest.fixture(scope="session")
-def gpu():
+def gpu(tmp_path_factory):
     import torch
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     torch.cuda.init()
+    # a process that dies in native code names the place
+    so = tmp_path_factory.mktemp("native") / "native_trace.so"
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", str(ROOT / "tests" / "native_trace.c"), "-o", str(so)],
+                   check=True)
+    ctypes.CDLL(str(so)).native_trace()
     return torch.device("cuda:0")
