@@ -119,6 +119,8 @@ class Compiled:
         self.calls = instr > self.opts.inline_limit
         self._bitplane()
 
+    emitted: Dict[str, int] = {}     # emit_source's choices (manifest)
+
     def _bitplane(self):
         """Bit-plane program (rtlflow_amd.bitplane) or None with the reason."""
         self.bitplane_blob = None
@@ -233,6 +235,11 @@ class Compiled:
             "block": self.opts.block,
             "form": "calls" if self.calls else "inline",
             "mw_waves": mw_waves(self),
+            # what emit_source chose: threads of the helped fused kernel (0:
+            # none), packed mtask kernels, batched kernel in its straight form
+            "help_threads": self.emitted.get("help_threads", 0),
+            "packed_mtasks": self.emitted.get("packed_mtasks", 0),
+            "straight_batched": self.emitted.get("straight_batched", False),
             "bitplane": self.bitplane_info,
             "streams": self.stream_table(),
         }
@@ -1590,6 +1597,8 @@ def _emit_source(comp: Compiled) -> str:
             parts[parts.index('#include "rf_stim.h"')] += '\n#include "rf_packed.h"'
         body = "\n".join(parts)
     hk, ht = emit_fused_help(comp)
+    comp.emitted = {"help_threads": ht, "packed_mtasks": sum("rf_pk_active" in pk for pk in packed.values()),
+                    "straight_batched": any("rf_k_persistent(" in pk for pk in packed.values())}
     if hk:
         body += "\n" + hk + "\n"
     parts = [body, emit_descriptor(comp, h, ht)]

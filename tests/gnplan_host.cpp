@@ -1,6 +1,7 @@
 // CPU model of the gate-net engine's LDS kernel: plans a program blob with
-// rf_gnplan.h and runs the wavefront programs over byte planes, one stimulus
-// per call. Built by tests/test_gnplan.py with the host compiler.
+// rf_gnplan.h for planes of ``pb`` bytes and runs the wavefront programs over
+// them, one stimulus at a time (one byte a plane: the plan's addresses divided
+// by its width). Built by tests/test_gnplan.py with the host compiler.
 #include <cstdlib>
 #include <cstring>
 #include <new>
@@ -46,17 +47,25 @@ extern "C" uint32_t gnplan_width(const uint32_t* h, uint32_t nwaves, uint64_t ld
     return pb;
 }
 
-// info[0..4]: slots, state slots, levels, wavefront rows, rows evaluated.
-// Returns 0, 1 when the program is not planned, 2 when a level's rows read a
-// slot that the same level writes, 3 when the wavefronts' barriers differ, 4
-// when a batch's row position is wrong, 5 when a class's operator is.
-extern "C" int gnplan_run(const uint32_t* h, uint32_t nwaves, uint64_t seed, const uint32_t* budgets, uint32_t n,
-                          uint64_t* hashes, uint32_t* info) {
+// info[0..6]: slots, state slots, levels, wavefront rows, rows evaluated,
+// wavefront rows of a batch, live RAMs. Returns 0, 1 when the program is not planned, 2
+// when a level's rows read a slot that the same level writes, 3 when the
+// wavefronts' barriers differ, 4 when a batch's row position is wrong, 5 when a
+// class's operator is, 6 when an address is no plane's.
+extern "C" int gnplan_run(const uint32_t* h, uint32_t nwaves, uint32_t pb, uint64_t seed, const uint32_t* budgets,
+                          uint32_t n, uint64_t* hashes, uint32_t* info) {
     Net net;
     if (!read_net(h, net)) return 1;
     Planner pl(net, nwaves);
     pl.schedule();
-    const Plan p = pl.emit(1);
+    const Plan p = pl.emit(pb);
+    info[5] = p.batch;
+    info[6] = p.n_ram_live;
+    bool off = false;
+    const auto at = [&](uint32_t address) {   // the plane's slot
+        if (address % pb || address / pb >= p.nslots) off = true;
+        return off ? 0u : address / pb;
+    };
     info[0] = p.nslots;
     info[1] = p.nstate;
     info[2] = p.levels;
@@ -96,7 +105,7 @@ extern "C" int gnplan_run(const uint32_t* h, uint32_t nwaves, uint64_t seed, con
                         for (uint32_t i = 0; i < n; ++i) {
                             const uint32_t to = p.batch == 1 ? i : i / 128 * 128 + 2 * (i % 64) + i % 128 / 64;
                             const uint64_t row = p.rows[per * (size_t)(wt[2] + ri[w]) + to];
-                            const uint32_t a = row & 0x3ffff, c = (row >> 18) & 0x3ffff, b = row >> 46;
+                            const uint32_t a = at(row & 0x3ffff), c = at((row >> 18) & 0x3ffff), b = at(row >> 46);
                             const uint32_t m = (row >> 36) & 63;
                             ++info[4];
                             read[a] = 1;
@@ -110,8 +119,9 @@ extern "C" int gnplan_run(const uint32_t* h, uint32_t nwaves, uint64_t seed, con
                             uint32_t v = cls == kMux ? (L[a] ? L[b] : L[c]) : op(m & 7, L[a], L[b]);
                             if (cls >= kOp && (m & 7) != op_bits(cls - kOp)) return 5;
                             if (cls == kPair) v = op(m >> 3, v, L[c]);
-                            L[d[1] + i] = v & 1;
-                            written[d[1] + i] = 1;
+                            const uint32_t to_slot = at(d[1] + i * pb);
+                            L[to_slot] = v & 1;
+                            written[to_slot] = 1;
                         }
                         ri[w] += (n + per - 1) / per;
                     }
@@ -123,23 +133,24 @@ extern "C" int gnplan_run(const uint32_t* h, uint32_t nwaves, uint64_t seed, con
                 if (rj[w] != p.words[4 * w + 1]) return 3;
             if (k) {
                 uint64_t v = 0;
-                for (uint32_t i = 0; i < n_po; ++i) v |= (uint64_t)L[p.words[p.off_po + i]] << i;
+                for (uint32_t i = 0; i < n_po; ++i) v |= (uint64_t)L[at(p.words[p.off_po + i])] << i;
                 const int nb = n_po <= 8 ? 1 : n_po <= 16 ? 2 : n_po <= 32 ? 4 : 8;
                 for (int i = 0; i < nb; ++i) hash = (hash ^ ((v >> (8 * i)) & 0xff)) * 0x100000001b3ull;
             }
             for (uint32_t r = 0; r < p.n_ram_live; ++r) {
                 const uint32_t* rw = &p.words[p.off_ram + r * p.ram_words];
                 uint64_t addr = 0, wd = 0;
-                for (uint32_t i = 0; i < ab; ++i) addr |= (uint64_t)L[rw[2 + i]] << i;
-                for (uint32_t i = 0; i < width; ++i) wd |= (uint64_t)L[rw[2 + ab + 1 + i]] << i;
+                for (uint32_t i = 0; i < ab; ++i) addr |= (uint64_t)L[at(rw[2 + i])] << i;
+                for (uint32_t i = 0; i < width; ++i) wd |= (uint64_t)L[at(rw[2 + ab + 1 + i])] << i;
                 uint64_t* m = &mem[(size_t)rw[0] * depth];
                 const uint64_t old = addr < depth ? m[addr] : 0;
-                if (L[rw[2 + ab]] && addr < depth) m[addr] = wd;
-                for (uint32_t i = 0; i < width; ++i) L[rw[1] + i] = (old >> i) & 1;
+                if (L[at(rw[2 + ab])] && addr < depth) m[addr] = wd;
+                for (uint32_t i = 0; i < width; ++i) L[at(rw[1] + i * pb)] = (old >> i) & 1;
             }
             for (uint32_t i = 0; i < n_pi; ++i) L[p.b0 + i] = L[p.a0 + i];
             gen(k + 1);
         }
+        if (off) return 6;
         hashes[s] = hash;
     }
     return 0;

@@ -11,6 +11,7 @@ from pathlib import Path
 import numpy as np
 import pytest
 
+import lds_nets
 import oracle
 from rtlflow_amd import gatenet as gn
 from rtlflow_amd.designs.netlist import MUX, GateTable, generate
@@ -27,10 +28,10 @@ def host(tmp_path_factory):
     return C.CDLL(str(so))
 
 
-def plan_run(host, prog, waves, seed, budgets):
+def plan_run(host, prog, waves, seed, budgets, pb=1):
     b = np.asarray(budgets, np.uint32)
-    out, info = np.zeros(len(b), np.uint64), np.zeros(5, np.uint32)
-    rc = host.gnplan_run(prog.ctypes.data_as(C.c_void_p), waves, C.c_uint64(seed), b.ctypes.data_as(C.c_void_p),
+    out, info = np.zeros(len(b), np.uint64), np.zeros(7, np.uint32)
+    rc = host.gnplan_run(prog.ctypes.data_as(C.c_void_p), waves, pb, C.c_uint64(seed), b.ctypes.data_as(C.c_void_p),
                          len(b), out.ctypes.data_as(C.c_void_p), info.ctypes.data_as(C.c_void_p))
     return rc, out, info
 
@@ -133,3 +134,35 @@ def test_plan_without_memory_is_no_plan(host):
         assert width(left) == 0, left
     assert width(total) == 4
     assert width(-1, lds=256) == 0
+
+
+@pytest.mark.parametrize("pb", [2, 4])
+@pytest.mark.parametrize("waves", [1, 16])
+def test_wider_planes_hash_as_the_oracle(host, pb, waves):
+    """Addresses and bank orders of 2- and 4-byte planes, batches of 4
+    wavefront rows (one wavefront) and of 1."""
+    batches = set()
+    for k in range(len(NETS)):
+        table = generate(seed=0x51A + k, **NETS[k])[1]
+        budgets = [7, 0, 12]
+        rc, got, info = plan_run(host, gn.program(table, threads=None), waves, 0xABCDEF, budgets, pb)
+        assert rc == 0
+        assert (got == oracle.netlist_run(table.to_bytes(), 0xABCDEF, len(budgets), budgets=budgets)).all()
+        batches.add(int(info[5]))
+    assert batches == ({1, 4} if waves == 1 else {1})
+
+
+@pytest.mark.parametrize("name", lds_nets.NETS)
+def test_instances_of_the_netlists_that_run_on_the_gpu(host, name):
+    """The plane width and the batches that each netlist of the GPU test plans
+    to, and its planned program against the oracle."""
+    width, batch, kw, _ = lds_nets.NETS[name]
+    table = lds_nets.table(name)
+    prog = gn.program(table, threads=None)
+    used = C.c_long(0)
+    assert host.gnplan_width(prog.ctypes.data_as(C.c_void_p), 16, C.c_uint64(lds_nets.LDS_BYTES), C.c_long(-1),
+                             C.byref(used)) == width
+    rc, got, info = plan_run(host, prog, 16, 5, [3, 1], width)
+    assert rc == 0 and info[5] == batch
+    assert info[6] > 14 or name != "20 RAMs"
+    assert (got == oracle.netlist_run(table.to_bytes(), 5, 2, budgets=[3, 1])).all()

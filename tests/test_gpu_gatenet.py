@@ -7,9 +7,10 @@ heuristic and the learned partitions."""
 import numpy as np
 import pytest
 
+import lds_nets
 import oracle
 from rtlflow_amd.designs import registry, rv32i
-from rtlflow_amd.gatenet import GateNet
+from rtlflow_amd.gatenet import GateNet, program
 
 SEED = registry.SEED_CFG[5]
 
@@ -71,6 +72,26 @@ def test_lds_form_matches_oracle(gpu, name, lanes, warm):
     for s0 in {0, lanes - k}:
         want = oracle.netlist_run(tb, SEED, k, stim0=s0, budgets=budgets[s0:s0 + k])
         assert (got[s0:s0 + k] == want).all(), s0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", lds_nets.NETS)
+def test_lds_instances_match_oracle(gpu, name):
+    """Every instance of the LDS kernel, and more RAMs than wavefronts for
+    them, against the oracle; a budget of 0 and a ragged last workgroup."""
+    table = lds_nets.table(name)
+    prog = program(table, threads=None)
+    lanes = 41
+    budgets = np.random.default_rng(7).integers(1, 30, size=lanes).astype(np.uint32)
+    budgets[[3, 40]] = 0
+    print(f"gatenet lds instance {name}", flush=True)
+    with GateNet(prog, lanes) as g:
+        # enough cycles that the handle plans
+        g.run(GateNet.BITPLANE, SEED, np.full(lanes, len(table.gate_type) // 512 + 1, np.uint32))
+        assert g.nodes_per_cycle(GateNet.BITPLANE) == 0
+        got, _ = g.run(GateNet.BITPLANE, SEED, budgets)
+    want = oracle.netlist_run(table.to_bytes(), SEED, lanes, budgets=budgets)
+    assert (got == want).all(), f"{int((got != want).sum())} of {lanes} differ"
 
 
 @pytest.mark.gpu

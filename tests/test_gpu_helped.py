@@ -47,3 +47,21 @@ def test_helped_done_lanes_and_chunks(gpu):
         _same(f, g, n)
         for lane in (5, 64, 100, 129, 130):
             assert f.lane_state(lane) == g.lane_state(lane), lane
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["gated", "kat_shift"])
+def test_helped_other_designs(gpu, name):
+    """A derived clock (three helpers) and wide operands (two): cut stages,
+    done lanes, launches of five cycles."""
+    cd = registry.get(name)
+    n = 130
+    done = np.zeros(n, np.uint8)
+    done[[0, 63, 64, 100, 129]] = 1
+    with cd.model(n, fused_chunk=5) as f, cd.model(n) as g:
+        for m, mode in ((f, MODE_FUSED), (g, MODE_GRAPH)):
+            m.begin(0xA3)
+            m.run_cycles(9, mode)
+            m.set_done(done)
+            m.run_cycles(17, mode)
+        _same(f, g, n)
