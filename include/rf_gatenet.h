@@ -25,8 +25,8 @@
  *                   over the first power-of-two count of groups that covers
  *                   every group with a lane still running (one graph per
  *                   count), so finished groups cost nothing.
- *                   Once a handle's cycles pay for the planning (about one
- *                   cycle per 512 gates), netlists whose live planes fit a
+ *                   Once a handle's cycles pay for the planning (cycles x
+ *                   launches a cycle reach a sixteenth of the gates), netlists whose live planes fit a
  *                   workgroup's LDS at 8, 16 or 32 stimuli per workgroup run
  *                   there instead: whole runs in one kernel, live gates only,
  *                   each workgroup to its own longest budget. The hashes are

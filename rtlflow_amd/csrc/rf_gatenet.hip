@@ -550,11 +550,14 @@ int check_program(const uint32_t* h, size_t words) {
     return RF_OK;
 }
 
-// When the LDS form is planned: the plan of a netlist of R records takes about
-// 0.13 us per record on the host (65 ms for the 500,000-gate net5) and saves
-// about 95 us per cycle there (122 us level by level, 26 us in LDS), so it has
-// paid after R / 700 cycles; the handle plans once its runs reach R / 512.
-constexpr uint64_t kPlanRecords = 512;
+// When the LDS form is planned: a plan takes about 0.17 us a record on the host
+// (82 ms for the 500,000 gates of net5, 0.9 ms for 5,500) and saves most of a
+// cycle's launches, about 3 us each (31 launches, 122 us level by level, 26 us
+// in LDS; 20 launches, 60 us and 5 us), so it has paid once cycles x launches
+// reach a seventeenth of the records: after 900 and 16 cycles. The handle plans
+// when its runs, the coming one included, reach a sixteenth.
+constexpr uint64_t kPlanShare = 16;
+uint64_t launches_per_cycle(const uint32_t* h) { return (uint64_t)h[H_LEV_FULL] + h[H_LEV_CONE] + 4; }
 
 // Plan the LDS form and load its tables. Leaves pb = 0 where that is not
 // possible (plan_program, or no device memory for the tables): the handle then
@@ -716,7 +719,7 @@ int rf_gn_run(rf_gatenet* g, uint32_t mode, uint64_t seed, const uint32_t* budge
     // the LDS form's plan, once this handle's cycles pay for it
     if (mode == RF_GN_BITPLANE && !g->planned) {
         g->cycles += ncyc;
-        if (g->cycles * kPlanRecords >= h[H_REC_FULL]) {
+        if (g->cycles * launches_per_cycle(h) * kPlanShare >= h[H_REC_FULL]) {
             g->planned = true;
             plan_lds(g);
         }

@@ -86,12 +86,24 @@ def test_lds_instances_match_oracle(gpu, name):
     budgets[[3, 40]] = 0
     print(f"gatenet lds instance {name}", flush=True)
     with GateNet(prog, lanes) as g:
-        # enough cycles that the handle plans
-        g.run(GateNet.BITPLANE, SEED, np.full(lanes, len(table.gate_type) // 512 + 1, np.uint32))
+        # enough cycles that the handle plans (four launches a cycle at least)
+        g.run(GateNet.BITPLANE, SEED, np.full(lanes, len(table.gate_type) // 64 + 1, np.uint32))
         assert g.nodes_per_cycle(GateNet.BITPLANE) == 0
         got, _ = g.run(GateNet.BITPLANE, SEED, budgets)
     want = oracle.netlist_run(table.to_bytes(), SEED, lanes, budgets=budgets)
     assert (got == want).all(), f"{int((got != want).sum())} of {lanes} differ"
+
+
+@pytest.mark.gpu
+def test_lds_form_begins_where_planning_pays(gpu):
+    """net5_small (6,000 gates, 24 launches a cycle) pays for its plan from 16
+    cycles on, the coming run's included."""
+    prog = registry.gatenet_program("net5_small")
+    print("gatenet lds net5_small planning", flush=True)
+    with GateNet(prog, 40) as g:
+        for cycles, planned in ((10, False), (5, False), (1, True), (3, True)):
+            g.run(GateNet.BITPLANE, SEED, np.full(40, cycles, np.uint32))
+            assert (g.nodes_per_cycle(GateNet.BITPLANE) == 0) == planned, cycles
 
 
 @pytest.mark.gpu
