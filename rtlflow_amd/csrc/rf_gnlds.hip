@@ -5,7 +5,7 @@
 // pass over the program, a workgroup barrier per level.
 //
 // Bound (net5: 178,000 live gates, 155,000 rows, 124 KB of planes at 8 stimuli
-// per workgroup, one workgroup per CU): LDS is busy 55 % of a cycle (half of
+// per workgroup, one workgroup per CU): LDS is busy 56 % of a cycle (half of
 // that bank conflicts), VALU issue 39 %, the vector cache 42 %; the rest is the
 // drain at 14 barriers: 26 us a cycle for 2,048 stimuli at once, against 122 us
 // for 4,096 level by level through HBM, where the 31 dependent launches of a
