@@ -648,6 +648,10 @@ extern "C" {
 int rf_gn_destroy(rf_gatenet* g) {
     if (!g) return RF_OK;
     if (g->stream) (void)hipStreamSynchronize(g->stream);
+    void* ps[] = {g->prog, g->P, g->X, g->M, g->hash, g->budget, g->ctl, g->sid, g->lwords, g->lrows, g->limage};
+    for (void* p : ps)
+        if (p) (void)hipFree(p);
+    // (after the frees, as rf_destroy)
     for (int k = 0; k < 2; ++k) {
         if (g->exec[k]) (void)hipGraphExecDestroy(g->exec[k]);
         if (g->graph[k]) (void)hipGraphDestroy(g->graph[k]);
@@ -656,9 +660,6 @@ int rf_gn_destroy(rf_gatenet* g) {
         if (g->bexec[k]) (void)hipGraphExecDestroy(g->bexec[k]);
         if (g->bgraph[k]) (void)hipGraphDestroy(g->bgraph[k]);
     }
-    void* ps[] = {g->prog, g->P, g->X, g->M, g->hash, g->budget, g->ctl, g->sid, g->lwords, g->lrows, g->limage};
-    for (void* p : ps)
-        if (p) (void)hipFree(p);
     if (g->e0) (void)hipEventDestroy(g->e0);
     if (g->e1) (void)hipEventDestroy(g->e1);
     if (g->stream) (void)hipStreamDestroy(g->stream);

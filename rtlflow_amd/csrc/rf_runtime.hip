@@ -671,7 +671,6 @@ int rf_destroy(rf_model* m) {
         (void)hipEventDestroy(q.e1);
     }
     for (hipEvent_t e : m->evfree) (void)hipEventDestroy(e);
-    drop_graphs(m);
     for (int c = 0; c < 4; ++c)
         if (m->cls[c]) (void)hipFree(m->cls[c]);
     void* ps[] = {m->mem, m->change, m->done, m->hash, m->cyc, m->stim, m->flags,
@@ -680,6 +679,9 @@ int rf_destroy(rf_model* m) {
         if (p) (void)hipFree(p);
     for (void* p : m->image_bufs)
         if (p) (void)hipFree(p);
+    // (after the frees, which wait for the whole device: the branches of a graph
+    // run on streams of HIP's own, not on m->stream)
+    drop_graphs(m);
     if (m->ev0) (void)hipEventDestroy(m->ev0);
     if (m->ev1) (void)hipEventDestroy(m->ev1);
     if (m->stream) (void)hipStreamDestroy(m->stream);
